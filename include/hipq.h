@@ -111,11 +111,13 @@ size_t hq_matmul_q_ws_bytes(int64_t M, int64_t N, int64_t K, int w_dtype);
  * w_dtype: one of the six GGUF formats Light fuses: HQ_Q4_0, HQ_Q5_0, HQ_Q8_0, HQ_Q4_K,
  * HQ_Q5_K or HQ_Q6_K, or HQ_Q6_K_R (a Q6_K weight after hq_repack_q6k).  K must be a
  * multiple of the block size.
- *  - M <= 8, Q4_K / Q5_K / Q6_K_R: the persistent int8-dot GEMV, x quantized to q8_1 inside its
+ *  - 3 <= M <= 16, Q4_K / Q5_K (from about 10M weights at M <= 8): f16 MFMA on exact integer weights,
+ *    x as one or two f16 parts under a power-of-two scale per row and 256 elements.
+ *  - Other M <= 8, Q4_K / Q5_K / Q6_K_R: the persistent int8-dot GEMV, x quantized to q8_1 inside its
  *    workgroups (K > 8192: into ws first).
  *  - M <= 8, Q8_0 / Q4_0 / Q5_0 / Q6_K: the LDS-staged int8-dot GEMV (x quantized in its
  *    workgroups up to K = 8192, into ws above).
- *  - M > 8 (K % 64 == 0): the bf16 MFMA GEMM; x is rounded to bf16 in ws; Q4_K tiles are
+ *  - Other M > 8 (K % 64 == 0): the bf16 MFMA GEMM; x is rounded to bf16 in ws; Q4_K tiles are
  *    dequantized inside the GEMM, the other formats once to a bf16 copy in ws.
  *  - M <= 8, rows longer than one GEMV team (Q4_K / Q5_K, 32768 < K <= 65536) or one LDS
  *    slice (the staged formats past 16 KB per row): x quantized into ws once, the GEMV over
@@ -165,9 +167,9 @@ int hq_matmul_q_gated(const float *x, const void *wg, const void *wu, float *out
 /* Gated projection that emits prepared activations for the next matmul:
  *   act_out (hq_act_bytes(M, N) bytes) = quantize_act(act(x @ dequant(wg)^T) * (x @ dequant(wu)^T)),
  * the same values hq_quantize_act would write for the F32 gated output.  N % 32 == 0.
- * For Q4_K / Q5_K with M <= 8 this is one kernel: the gated GEMV quantizes each completed
- * 32-row chunk of its output in the epilogue (the first launch of hq_mlp_q).  Other cases
- * run hq_matmul_q_gated into ws, then the quantizer.  Feed act_out to hq_matmul_q_act (the
+ * For Q4_K / Q5_K with M <= 2 (and small weights to M <= 8) this is one kernel: the gated GEMV
+ * quantizes each completed 32-row chunk of its output in the epilogue (the first launch of
+ * hq_mlp_q).  Other cases run hq_matmul_q_gated into ws, then the quantizer.  Feed act_out to hq_matmul_q_act (the
  * down projection).  Light: models/llama.go:1306-1328 (gate, up, SiLU * up before
  * DownProj); no counterpart op in Light. */
 size_t hq_matmul_q_gated_act_ws_bytes(int64_t M, int64_t N, int64_t K, int w_dtype);
@@ -177,9 +179,10 @@ int hq_matmul_q_gated_act(const float *x, const void *wg, const void *wu, void *
 /* The gated MLP block of a decoder layer:
  *   out (M, H) F32 = (act(x @ dequant(wg)^T) * (x @ dequant(wu)^T)) @ dequant(wd)^T
  * with x (M, H) F32, wg and wu (I, H), wd (H, I), all of w_dtype; act as above.
- * For Q4_K with M <= 8 this is two launches: the gated gate/up GEMV, which writes its
- * output already quantized for the next matmul into ws, and the down GEMV on it.  Other
- * cases run hq_matmul_q_gated into ws and then hq_matmul_q.
+ * For Q4_K with M <= 8 this is hq_matmul_q_gated_act followed by hq_matmul_q_act, bit for bit: at
+ * M <= 2 (and for small weights) two launches, the gated gate/up GEMV, which writes its output
+ * already quantized for the next matmul into ws, and the down GEMV on it.  Other cases run
+ * hq_matmul_q_gated into ws and then hq_matmul_q.
  * Light: models/llama.go:1306-1333 (GatedLinear or MatMulQ/SiLU/Mul, then DownProj).
  * No counterpart op in Light. */
 size_t hq_mlp_q_ws_bytes(int64_t M, int64_t H, int64_t I, int w_dtype);
@@ -203,7 +206,9 @@ int hq_mlp_q(const float *x, const void *wg, const void *wu, const void *wd, flo
  * GEMVs use both levels.  The layout is internal and may change with the version. */
 size_t hq_act_bytes(int64_t M, int64_t K);
 int hq_quantize_act(const void *x, int x_dtype, void *act, int64_t M, int64_t K, hq_stream_t stream);
-/* Workspace hq_matmul_q_act needs beyond the act buffer (0 for the GEMV). */
+/* Workspace hq_matmul_q_act uses beyond the act buffer.  For Q4_K / Q5_K at 3 <= M <= 8 with rows
+ * past 4096 it is optional: without it (a smaller ws, or a library workspace that cannot grow
+ * during capture) the int8 GEMV serves the call. */
 size_t hq_matmul_q_act_ws_bytes(int64_t M, int64_t N, int64_t K, int w_dtype);
 /* out (M, N) F32 = x @ dequant(w)^T from prepared activations.  For M <= 8, and for
  * any M when K is not a multiple of 64, the weight must take the int8 GEMV (16-byte
@@ -254,7 +259,8 @@ size_t hq_int4_matmul_ws_bytes(int64_t M, int64_t N, int64_t K, int G, int x_dty
  * quant/int4.go:11-34): codes U32 (N, K/8), nibble j of word c = W[n, 8c+j];
  * scales / zeros F32 (N, K/G); W = s * (code - z).  x_dtype F32, BF16 or F16;
  * y has x's dtype (F16 is an extension: Light takes F32 or BF16, ops/int4.go:70-72).
- * K % 32 == 0 and G % 32 == 0.  M <= 8 (or G % 64 != 0): x is quantized to q8_1
+ * K % 32 == 0 and G % 32 == 0.  3 <= M <= 16, G % 128 == 0 and large weights: f16 MFMA on the exact
+ * codes, F32 x as two f16 parts (16-bit x is exact in one).  Other M <= 8 (or G % 64 != 0): x is quantized to q8_1
  * into ws and the int8-dot GEMV runs (K <= 65536; rows past 32768 with 256 % G == 0 as two
  * K halves whose F32 partials are summed in ws); otherwise -- and for longer rows at
  * any M when G % 64 == 0 -- the MFMA GEMMs run (F16 x at 8 < M <= 64 as given, else

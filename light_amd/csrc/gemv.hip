@@ -1170,14 +1170,15 @@ static size_t gemm_ws(int64_t M, int64_t N, int64_t K, int dt) {
 
 size_t matmul_q_ws_bytes(int64_t M, int64_t N, int64_t K, int dt) {
   if (M <= 0 || K <= 0 || K % 32) return 0;
-  if (use_gemm(M, dt) && gemm_k_ok(K)) return gemm_ws(M, N, K, dt);
+  const size_t sk = dt == Q4_K || dt == Q5_K ? skinny_ws_bytes(M, K, false) : 0;
+  if (use_gemm(M, dt) && gemm_k_ok(K)) return std::max(sk, gemm_ws(M, N, K, dt));
   // Long Q4_K / Q5_K rows: x quantized once, then the second K half's outputs.
   if ((dt == Q4_K || dt == Q5_K) && K > 32768 && K <= 65536 && K % 256 == 0)
-    return std::max((size_t)(al256(act_bytes(M, K)) + 4 * M * N), q4kx_halves_x_ws_bytes(M, N, K));
+    return std::max(sk, std::max((size_t)(al256(act_bytes(M, K)) + 4 * M * N), q4kx_halves_x_ws_bytes(M, N, K)));
   // Long staged rows (split into K parts): the parts' outputs as well.
   if ((dt == Q8_0 || dt == Q4_0 || dt == Q5_0 || dt == Q6_K) && staged_row_bytes(dt, K) + 16 > 16384)
     return std::max((size_t)(al256(act_bytes(M, K)) + 4 * M * N), staged_parts_x_ws_bytes(dt, M, N, K));
-  return (size_t)act_bytes(M, K);
+  return std::max(sk, (size_t)act_bytes(M, K));
 }
 
 // Long rows split into K parts (act_long_rows_ok) need the later parts' outputs.
@@ -1189,7 +1190,12 @@ static bool long_rows_dt(int64_t K, int dt) {
 size_t matmul_act_ws_bytes(int64_t M, int64_t N, int64_t K, int dt) {
   if (M <= 0 || K <= 0 || K % 32) return 0;
   if (use_gemm(M, dt) && gemm_k_ok(K)) return gemm_ws(M, N, K, dt);
-  return long_rows_dt(K, dt) && N > 0 ? (size_t)(4 * M * N) : 0;
+  if (long_rows_dt(K, dt)) return N > 0 ? (size_t)(4 * M * N) : 0;
+  return dt == Q4_K || dt == Q5_K ? skinny_ws_bytes(M, K, false) : 0;
+}
+
+bool matmul_act_ws_optional(int64_t M, int64_t K, int dt) {
+  return !(use_gemm(M, dt) && gemm_k_ok(K)) && !long_rows_dt(K, dt);
 }
 
 bool act_long_rows_ok(int64_t M, int64_t N, int64_t K, int dt, const void *w, const void *act) {
@@ -1220,11 +1226,14 @@ int launch_matmul_act(const void *act, const void *w, float *out, int64_t M, int
     return launch_staged_parts(act, w, out, static_cast<float *>(ws), M, N, K, dt, s);
   if (q4kx_halves_ok(M, N, K, dt, w, act))
     return launch_gemv_q4kx_act_halves(act, w, out, static_cast<float *>(ws), M, N, K, dt, s);
+  if (M <= kGemvMaxRows && skinny_ok(M, N, K, dt, w, act) && (ws || skinny_ws_bytes(M, K, false) == 0))
+    return launch_skinny_act(act, true, w, out, M, N, K, dt, ws, s);
   return launch_gemv_act(act, w, out, M, N, K, dt, s);
 }
 
 int launch_matmul_q(const float *x, const void *w, float *out, int64_t M, int64_t N, int64_t K, int dt, void *ws,
                     hipStream_t s) {
+  if (skinny_ok(M, N, K, dt, w, x)) return launch_skinny(x, w, nullptr, out, M, N, K, 0, dt, ws, s);
   if (use_gemm(M, dt) && gemm_k_ok(K)) return run_gemm(x, false, w, out, M, N, K, dt, ws, s);
   if (dt == Q6_K_R) {
     // The planar Q6_K layout is only read by the team GEMV (and dequantized for the GEMM).

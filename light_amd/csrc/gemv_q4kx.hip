@@ -2485,6 +2485,7 @@ size_t matmul_q_gated_ws_bytes(int64_t M, int64_t N, int64_t K, int dt) {
 
 int launch_matmul_q_gated(const float *x, const void *wg, const void *wu, float *out, int64_t M, int64_t N, int64_t K,
                           int dt, int act, void *ws, hipStream_t s) {
+  if (skinny_gated_ok(M, N, K, dt, wg, wu, x)) return launch_skinny(x, wg, wu, out, M, N, K, act, dt, ws, s);
   if (q4kx_ok(M, N, K, wg, wu, x, dt)) {
     if (q4kx_xin(K)) return launch_gemv_q4kx(x, wg, wu, out, M, N, K, act, dt, s);
     Q4kxArgs a;
@@ -2665,7 +2666,8 @@ static int run_gate_cu(const Q4kxArgs &a, hipStream_t s) {
 int launch_matmul_q_gated_act(const float *x, const void *wg, const void *wu, uint8_t *aout, int64_t M, int64_t N,
                               int64_t K, int dt, int act, void *ws, hipStream_t s) {
   int P, TP, RW;
-  if (N % 256 == 0 && q4kx_ok(M, N, K, wg, wu, x, dt) && q4kx_geom(K, 256, &P, &TP, &RW) && 32 % RW == 0) {
+  const bool skinny = skinny_gated_ok(M, N, K, dt, wg, wu, x);  // (the unfused path below)
+  if (!skinny && N % 256 == 0 && q4kx_ok(M, N, K, wg, wu, x, dt) && q4kx_geom(K, 256, &P, &TP, &RW) && 32 % RW == 0) {
     Q4kxArgs a;
     if (int rc = q4kx_setup(a, M, N, K, 256, q4kx_row_bytes(dt, K), "matmul_q_gated_act")) return rc;
     a.x = x;
@@ -2688,11 +2690,23 @@ int launch_matmul_q_gated_act(const float *x, const void *wg, const void *wu, ui
 int launch_mlp_q(const float *x, const void *wg, const void *wu, const void *wd, float *out, int64_t M, int64_t H,
                  int64_t I, int dt, int act, void *ws, hipStream_t s) {
   if (mlp_fused_ok(M, H, I, dt, wg, wu, wd, x)) {
+    // hq_matmul_q_gated_act followed by hq_matmul_q_act, bit for bit: each half on the kernel that
+    // call would take.
+    auto *hact = static_cast<uint8_t *>(ws);
+    void *rest = static_cast<char *>(ws) + al256(4 * M * I);
+    if (skinny_gated_ok(M, I, H, dt, wg, wu, x)) {
+      float *h = static_cast<float *>(ws);
+      if (int rc = launch_skinny(x, wg, wu, h, M, I, H, act, dt, rest, s)) return rc;
+      // (The down projection's conversion of x takes h through its quantization itself.)
+      if (skinny_ok(M, H, I, dt, wd, h)) return launch_skinny_act(h, false, wd, out, M, H, I, dt, rest, s);
+      if (int rc = launch_quantize_act(h, F32, rest, M, I, s)) return rc;
+      return launch_gemv_q4kx_act(rest, wd, out, M, H, I, dt, s);
+    }
     // Launch 1: gated gate/up on x, output quantized straight into ws (act layout of (M, I)).
-    auto *h = static_cast<uint8_t *>(ws);
-    if (int rc = launch_matmul_q_gated_act(x, wg, wu, h, M, I, H, dt, act, nullptr, s)) return rc;
+    if (int rc = launch_matmul_q_gated_act(x, wg, wu, hact, M, I, H, dt, act, nullptr, s)) return rc;
     // Launch 2: down projection on the prepared h.
-    return launch_gemv_q4kx_act(h, wd, out, M, H, I, dt, s);
+    if (skinny_ok(M, H, I, dt, wd, hact)) return launch_skinny_act(hact, true, wd, out, M, H, I, dt, rest, s);
+    return launch_gemv_q4kx_act(hact, wd, out, M, H, I, dt, s);
   }
   float *h = static_cast<float *>(ws);
   void *inner = static_cast<char *>(ws) + al256(4 * M * I);

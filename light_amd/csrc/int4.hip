@@ -278,8 +278,7 @@ static void run_i4_m(const I4Args &a, int mm, hipStream_t s) {
 // x rows past M are clamped and their stores masked).
 static bool int4_gemm_ok(int64_t M, int64_t K, int G) { return (M > 8 || K / 32 > 2048) && G % 64 == 0; }
 
-size_t int4_ws_bytes(int64_t M, int64_t N, int64_t K, int G, int x_dtype) {
-  if (M <= 0 || K <= 0 || K % 32) return 0;
+static size_t int4_ws(int64_t M, int64_t N, int64_t K, int G, int x_dtype) {
   if (!int4_gemm_ok(M, K, G)) {
     // Long rows (two K halves): the halves' F32 partials as well.
     const bool halves = M <= 8 && K > 32768 && K <= 65536 && K % 256 == 0 && G > 0 && 256 % G == 0;
@@ -293,6 +292,11 @@ size_t int4_ws_bytes(int64_t M, int64_t N, int64_t K, int G, int x_dtype) {
   return (x_dtype == BF16 ? 0 : gemm_x_bytes(M, K)) + gemm_partial_bytes(M, N, K, x_dtype == F32);
 }
 
+size_t int4_ws_bytes(int64_t M, int64_t N, int64_t K, int G, int x_dtype) {
+  if (M <= 0 || K <= 0 || K % 32) return 0;
+  return std::max(skinny_ws_bytes(M, K, true), int4_ws(M, N, K, G, x_dtype));
+}
+
 int launch_int4_matmul(const void *x, int x_dtype, const uint32_t *codes, const float *s, const float *z, void *y,
                        int64_t M, int64_t N, int64_t K, int G, void *ws, hipStream_t st) {
   if (N > INT32_MAX || K > INT32_MAX) return fail(HQ_EUNSUPPORTED, "int4_matmul", "N or K too large");
@@ -301,6 +305,8 @@ int launch_int4_matmul(const void *x, int x_dtype, const uint32_t *codes, const 
     // all of K, no split-K partials.
     return launch_i4cu(static_cast<const uint16_t *>(x), codes, s, z, y, M, N, K, G, st);
   }
+  if (skinny_int4_ok(M, N, K, G, x_dtype, codes, x))
+    return launch_skinny_int4(x, x_dtype, codes, s, z, y, M, N, K, G, ws, st);
   if (int4_gemm_ok(M, K, G) && i4f16_small_ok(M, N, K, G, x_dtype, x, codes)) {
     // F16 x at M <= 64: the exact-weight f16 MFMA kernel reads x as given.
     return launch_i4f16_small(static_cast<const uint16_t *>(x), codes, s, z, y,

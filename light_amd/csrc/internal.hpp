@@ -50,6 +50,8 @@ int launch_gemm_ws_bf16(const uint16_t *xb, const uint16_t *wb, float *out, floa
                         int64_t K, hipStream_t s);
 size_t matmul_q_ws_bytes(int64_t M, int64_t N, int64_t K, int dt);
 size_t matmul_act_ws_bytes(int64_t M, int64_t N, int64_t K, int dt);
+// hq_matmul_q_act can do without that workspace (the int8 GEMV in place of skinny.hip).
+bool matmul_act_ws_optional(int64_t M, int64_t K, int dt);
 int launch_matmul_q(const float *x, const void *w, float *out, int64_t M, int64_t N, int64_t K, int dt, void *ws,
                     hipStream_t s);
 const char *matmul_q_kernel_name(int64_t M, int dt);
@@ -97,6 +99,21 @@ int launch_gemv_q4kx_act(const void *act_in, const void *w, float *out, int64_t 
 // Q4_K / Q5_K rows of 32768 < K <= 65536 at M <= 8: the act GEMV on each K half, then an add
 // (tmp: M * N floats).
 bool q4kx_halves_ok(int64_t M, int64_t N, int64_t K, int dt, const void *w, const void *act);
+// The f16 MFMA product for a few rows of x (skinny.hip): Q4_K / Q5_K (w1 != NULL: gated) and
+// int4.  ws: skinny_ws_bytes (rows past 8192 only).
+constexpr int64_t kSkinnyMaxRows = 16;
+// (A row's x record stays below 1 MiB, the library workspace's first size.)
+constexpr int64_t kSkinnyMaxK = 29696;
+bool skinny_ok(int64_t M, int64_t N, int64_t K, int dt, const void *w, const void *x);
+bool skinny_gated_ok(int64_t M, int64_t N, int64_t K, int dt, const void *wg, const void *wu, const void *x);
+bool skinny_int4_ok(int64_t M, int64_t N, int64_t K, int G, int x_dtype, const void *codes, const void *x);
+size_t skinny_ws_bytes(int64_t M, int64_t K, bool int4);
+int launch_skinny(const float *x, const void *w0, const void *w1, float *out, int64_t M, int64_t N, int64_t K, int act,
+                  int dt, void *ws, hipStream_t s);
+int launch_skinny_act(const void *x, bool prepared, const void *w, float *out, int64_t M, int64_t N, int64_t K, int dt,
+                      void *ws, hipStream_t s);
+int launch_skinny_int4(const void *x, int x_dtype, const uint32_t *codes, const float *sc, const float *zr, void *y,
+                       int64_t M, int64_t N, int64_t K, int G, void *ws, hipStream_t s);
 // The Q4_K / Q5_K halves for M >= 2 rows of F32 x: one launch per half for every row of x.
 size_t q4kx_halves_x_ws_bytes(int64_t M, int64_t N, int64_t K);
 int launch_gemv_q4kx_halves_x(const float *x, const void *w, float *out, void *ws, int64_t M, int64_t N, int64_t K,

@@ -1,0 +1,116 @@
+"""The f16 MFMA product for 3 to 16 rows of x (skinny.hip) against float64 on the dequantized weight.
+
+Bounds, relative to |w_n| |x_m| (Cauchy-Schwarz on the rounding of x; the weights are exact
+integers and f32 scales): one f16 part of x is 2^-12 per element, so 2.5e-4 with the f32 sums;
+two parts are 2^-22, which leaves the f32 sums' 2e-5; 16-bit x is exact in one part, so its output
+rounding (bf16 2^-9, f16 2^-11 of |y| <= |w| |x|) is what shows.
+"""
+import pytest
+import torch
+
+from light_amd import hipq, synth
+
+pytestmark = pytest.mark.gpu
+
+
+def _x(M, K, dev, seed):
+    """N(0, 1) rows; row 0 with outliers and a zero stretch, row 1 tiny, row 2 huge."""
+    g = torch.Generator(device=dev).manual_seed(seed)
+    x = torch.randn(M, K, device=dev, generator=g)
+    x[0, ::97] *= 40.0
+    x[0, 256:512] = 0.0
+    x[1] *= 1e-20
+    x[2] *= 1e20
+    return x
+
+
+def _weight(dt, N, K, dev, seed):
+    w = torch.from_numpy(synth.gguf_weight(dt, N, K, synth.rng(seed))).to(dev)
+    return w, hipq.dequant(w, N * K, dt).view(N, K).double()
+
+
+def _err(y, want, x, wd):
+    scale = torch.outer(x.double().norm(dim=1), wd.norm(dim=1))
+    return ((y.double() - want).abs() / scale).max().item()
+
+
+# (N, K): tile and group remainders of the resident kernel (K <= 4096; 16, 15, 8 and 2 groups), then
+# of the long one (17 groups: two chunks of 9 and 8; one tile, two tiles and four per workgroup).
+SHAPES = [(2567, 4096), (2640, 3840), (5008, 2048), (20011, 512), (2440, 4352), (1536, 14336), (5000, 4608),
+          (10000, 5120), (1600, 16640)]
+
+
+@pytest.mark.parametrize("dt", [hipq.Q4_K, hipq.Q5_K])
+@pytest.mark.parametrize("M", [3, 4, 5, 8, 9, 16])
+@pytest.mark.parametrize("N,K", SHAPES)
+def test_matmul_q(dev, dt, M, N, K):
+    print(f"[case] skinny dt={hipq.NAMES[dt]} M={M} N={N} K={K}", flush=True)
+    w, wd = _weight(dt, N, K, dev, seed=N + K)
+    x = _x(M, K, dev, seed=M)
+    y = hipq.matmul_q(x, w, N, K, dt)
+    pair = M <= 8 and (K < 4096 or K > 16384)
+    assert _err(y, x.double() @ wd.t(), x, wd) <= (2e-5 if pair else 2.5e-4)
+    assert torch.equal(y, hipq.matmul_q(x, w, N, K, dt)), "not deterministic"
+
+
+@pytest.mark.parametrize("M", [9, 16])
+@pytest.mark.parametrize("N,K", [(1, 256), (17, 256), (40, 768), (100, 8192)])
+def test_small_weights(dev, M, N, K):
+    print(f"[case] skinny small M={M} N={N} K={K}", flush=True)
+    w, wd = _weight(hipq.Q4_K, N, K, dev, seed=K)
+    x = _x(M, K, dev, seed=M)
+    assert _err(hipq.matmul_q(x, w, N, K, hipq.Q4_K), x.double() @ wd.t(), x, wd) <= 2.5e-4
+
+
+@pytest.mark.parametrize("dt", [hipq.Q4_K, hipq.Q5_K])
+@pytest.mark.parametrize("M,N,K", [(3, 2567, 4096), (8, 5008, 2048), (16, 1000, 3840), (5, 1608, 6400), (12, 6000, 4352)])
+def test_gated(dev, dt, M, N, K):
+    print(f"[case] skinny gated dt={hipq.NAMES[dt]} M={M} N={N} K={K}", flush=True)
+    (wg, g), (wu, u) = _weight(dt, N, K, dev, seed=N), _weight(dt, N, K, dev, seed=N + 1)
+    x = torch.randn(M, K, device=dev, generator=torch.Generator(device=dev).manual_seed(M)) * 0.01
+    h = hipq.matmul_q_gated(x, wg, wu, N, K, dt)
+    a, b = x.double() @ g.t(), x.double() @ u.t()
+    # The product rule on the plain bound (|silu'| <= 1.1), and f32's exp.
+    xn, gn, un = x.double().norm(dim=1)[:, None], g.norm(dim=1)[None, :], u.norm(dim=1)[None, :]
+    silu = torch.nn.functional.silu(a)
+    bound = 2.5e-4 * xn * (1.1 * gn * b.abs() + un * silu.abs()) + 1e-5 * (silu * b).abs() + 1e-7 * xn * xn * gn * un
+    assert ((h.double() - silu * b).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("M,H,I", [(3, 4096, 5120), (5, 2048, 8192), (8, 4096, 3072), (6, 8192, 2048), (4, 2048, 8192)])
+def test_mlp_equals_its_halves(dev, M, H, I):
+    """Each half of the block on the kernel its own call takes, whichever those are."""
+    print(f"[case] skinny mlp M={M} H={H} I={I}", flush=True)
+    (wg, _), (wu, _), (wd, _) = (_weight(hipq.Q4_K, r, c, dev, seed=i) for i, (r, c) in enumerate(((I, H), (I, H), (H, I))))
+    x = torch.randn(M, H, device=dev, generator=torch.Generator(device=dev).manual_seed(M)) * 0.01
+    want = hipq.matmul_q_act(hipq.matmul_q_gated_act(x, wg, wu, I, H, hipq.Q4_K), wd, M, H, I, hipq.Q4_K)
+    assert torch.equal(hipq.mlp_q(x, wg, wu, wd, H, I, hipq.Q4_K), want)
+
+
+@pytest.mark.parametrize("M,N,K", [(3, 2567, 4096), (8, 1536, 14336)])
+def test_prepared_without_workspace(dev, M, N, K):
+    """hq_matmul_q_act with a caller's workspace too small for x's records takes the int8 GEMV."""
+    print(f"[case] skinny act M={M} N={N} K={K}", flush=True)
+    w, wd = _weight(hipq.Q4_K, N, K, dev, seed=K)
+    x = torch.randn(M, K, device=dev, generator=torch.Generator(device=dev).manual_seed(M))
+    act = hipq.quantize_act(x)
+    y = hipq.matmul_q_act(act, w, M, N, K, hipq.Q4_K)
+    small = hipq.matmul_q_act(act, w, M, N, K, hipq.Q4_K, ws=torch.empty(16, dtype=torch.uint8, device=dev))
+    want = x.double() @ wd.t()
+    assert _err(y, want, x, wd) <= 3e-4 and _err(small, want, x, wd) <= 1e-3
+
+
+@pytest.mark.parametrize("xdt,tol", [(torch.float32, 2e-5), (torch.bfloat16, 2.0 ** -8), (torch.float16, 2.0 ** -10)])
+@pytest.mark.parametrize("M", [3, 8, 16])
+@pytest.mark.parametrize("N,K,G", [(3208, 4096, 128), (3600, 3584, 256), (5000, 2688, 128), (4100, 4224, 128),
+                                   (2056, 18944, 128), (4104, 8192, 512)])
+def test_int4(dev, xdt, tol, M, N, K, G):
+    print(f"[case] skinny int4 x={xdt} M={M} N={N} K={K} G={G}", flush=True)
+    codes, s, z = (torch.from_numpy(a).to(dev) for a in synth.int4_weight(N, K, G, synth.rng(N + K)))
+    z = z + 0.25  # fractional zero points
+    codes = codes.view(torch.int32)
+    x = torch.randn(M, K, device=dev, generator=torch.Generator(device=dev).manual_seed(M)).to(xdt)
+    y = hipq.int4_matmul(x, codes, s, z, G)
+    wd = hipq.int4_dequant(codes, s, z, G).double()
+    # (M > 8 below the rule's size takes the bf16 GEMM: both operands rounded, 2^-8.)
+    assert _err(y, x.double() @ wd.t(), x, wd) <= (tol if M <= 8 else max(tol, 2.0 ** -8 + tol))

@@ -66,9 +66,10 @@ struct WsArgs {
   const uint16_t *x;   // bf16 [M][K]
   const uint8_t *w;    // Q4_K blocks (N, K) or int4 codes (N, K/8)
   const float *s, *z;  // int4 scales / zeros (N, K/G)
-  float *out;          // [M][N] or split partials [S][M][N]
+  void *out;           // [M][N] of ODT (one split), or F32 split partials [S][M][N]
   int M, N, K, G;
   int tiles_m, tiles_n, splits, xcd_map;
+  int gpr, gsh;        // int4: groups per row; log2(G), or -1
   int64_t row_bytes;
 };
 
@@ -128,7 +129,7 @@ struct WsInt4 {
     dma16(a.w + (int64_t)r * (a.K / 2) + (k0 >> 1) + 16 * (lane >> 5), dst);
     int r2 = row_base + (lane & 31);
     r2 = r2 < a.N ? r2 : a.N - 1;
-    const int64_t gi = (int64_t)r2 * (a.K / a.G) + k0 / a.G;
+    const int64_t gi = (int64_t)r2 * a.gpr + (a.gsh >= 0 ? k0 >> a.gsh : k0 / a.G);
     dma4(lane < 32 ? (const void *)(a.s + gi) : (const void *)(a.z + gi), dst + 1024);
   }
   // Thread (row r, half h): codes bytes [16h, 16h+16) = k 32h + i, i < 32 (nibble order).
@@ -137,17 +138,21 @@ struct WsInt4 {
                                  float out_hi[16]) {
     const u32x4 q = *reinterpret_cast<const u32x4 *>(raw + (32 * h + r) * 16);
     const float s = reinterpret_cast<const float *>(raw + 1024)[r];
-    const float z = reinterpret_cast<const float *>(raw + 1024)[32 + r];
+    // s q - s z in one FMA, the quants as bytes (one mask per four, v_cvt_f32_ubyteN): the weight
+    // is rounded to bf16 next, so this is not the bit-exact dequant.
+    const float nz = -s * reinterpret_cast<const float *>(raw + 1024)[32 + r];
 #pragma unroll
-    for (int k = 0; k < 4; k++)
+    for (int k = 0; k < 4; k++) {
+      const uint32_t ev = q[k] & 0x0F0F0F0Fu, od = (q[k] >> 4) & 0x0F0F0F0Fu;
 #pragma unroll
       for (int j = 0; j < 8; j++) {
-        const float v = s * ((float)((q[k] >> (4 * j)) & 15) - z);
+        const float v = __fmaf_rn(s, (float)((((j & 1) ? od : ev) >> (8 * (j >> 1))) & 0xffu), nz);
         if (k < 2)
           out_lo[8 * k + j] = v;
         else
           out_hi[8 * (k - 2) + j] = v;
       }
+    }
   }
 };
 
@@ -169,7 +174,9 @@ struct WsBf16 {
   __device__ static void dequant(const WsArgs &, const uint8_t *, int, int, int, float *, float *) {}
 };
 
-template <class WF, int BM>
+// ODT: the output's dtype.  BF16 / F16 are stored by the tile's own epilogue when K is not split
+// (int4 18944 x 3584, BF16, M = 2048: F32 partials and their conversion launch cost 40 of 405 us).
+template <class WF, int BM, int ODT>
 __global__ __launch_bounds__(512) void gemm_ws_kernel(WsArgs a) {
   using T = WsTile<BM, WF>;
   extern __shared__ __align__(16) uint8_t smem[];
@@ -314,7 +321,7 @@ __global__ __launch_bounds__(512) void gemm_ws_kernel(WsArgs a) {
       __syncthreads();
     }
     // Epilogue: lane holds D[8*(r/4) + 4*(lane/32) + r%4][lane%32] of each 32x32 tile.
-    float *out = a.out + (int64_t)blockIdx.z * a.M * a.N;
+    const int64_t z0 = (int64_t)blockIdx.z * a.M * a.N;
 #pragma unroll
     for (int i = 0; i < T::MT; i++)
 #pragma unroll
@@ -324,7 +331,14 @@ __global__ __launch_bounds__(512) void gemm_ws_kernel(WsArgs a) {
 #pragma unroll
         for (int r = 0; r < 16; r++) {
           const int row = m0 + (wm * T::MT + i) * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-          if (row < a.M) out[(int64_t)row * a.N + col] = acc[i][j][r];
+          if (row >= a.M) continue;
+          const int64_t o = z0 + (int64_t)row * a.N + col;
+          if constexpr (ODT == F32)
+            static_cast<float *>(a.out)[o] = acc[i][j][r];
+          else if constexpr (ODT == BF16)
+            static_cast<uint16_t *>(a.out)[o] = f2bf_rne(acc[i][j][r]);
+          else
+            static_cast<uint16_t *>(a.out)[o] = f2h_rne(acc[i][j][r]);
         }
       }
   }
@@ -343,20 +357,21 @@ static int ws_splits(int64_t M, int64_t N, int64_t K) {
 }
 
 size_t gemm_ws_partial_bytes(int64_t M, int64_t N, int64_t K, bool f32_out) {
+  (void)f32_out;
   const int s = ws_splits(M, N, K);
-  return (s > 1 || !f32_out) ? (size_t)s * (size_t)M * (size_t)N * 4 : 0;
+  return s > 1 ? (size_t)s * (size_t)M * (size_t)N * 4 : 0;
 }
 
 int launch_splitk_reduce(const float *part, void *out, int out_dtype, int64_t n, int splits, hipStream_t s);
 
-template <class WF, int BM>
-static int launch_ws_t(WsArgs a, int out_dtype, void *out, float *partials, hipStream_t s) {
+template <class WF, int BM, int ODT>
+static int launch_ws_o(WsArgs a, hipStream_t s) {
   using T = WsTile<BM, WF>;
   static bool attr_set[64] = {false};
   int dev = 0;
   (void)hipGetDevice(&dev);
   if (dev >= 0 && dev < 64 && !attr_set[dev]) {
-    if (int rc = check(hipFuncSetAttribute((const void *)gemm_ws_kernel<WF, BM>,
+    if (int rc = check(hipFuncSetAttribute((const void *)gemm_ws_kernel<WF, BM, ODT>,
                                            hipFuncAttributeMaxDynamicSharedMemorySize, T::LDS),
                        "hipFuncSetAttribute"))
       return rc;
@@ -364,15 +379,26 @@ static int launch_ws_t(WsArgs a, int out_dtype, void *out, float *partials, hipS
   }
   a.tiles_m = (int)cdiv(a.M, BM);
   a.tiles_n = (int)cdiv(a.N, WBN);
-  a.splits = ws_splits(a.M, a.N, a.K);
   const int ntiles = a.tiles_m * a.tiles_n;
   a.xcd_map = ntiles % 8 == 0;
-  const bool direct = a.splits == 1 && out_dtype == F32;
-  a.out = direct ? static_cast<float *>(out) : partials;
   dim3 grid((unsigned)ntiles, 1, (unsigned)a.splits);
-  gemm_ws_kernel<WF, BM><<<grid, 512, T::LDS, s>>>(a);
-  if (int rc = check_launch("gemm_ws")) return rc;
-  if (direct) return HQ_OK;
+  gemm_ws_kernel<WF, BM, ODT><<<grid, 512, T::LDS, s>>>(a);
+  return check_launch("gemm_ws");
+}
+
+template <class WF, int BM>
+static int launch_ws_t(WsArgs a, int out_dtype, void *out, float *partials, hipStream_t s) {
+  a.splits = ws_splits(a.M, a.N, a.K);
+  if (a.splits == 1) {
+    a.out = out;
+    if constexpr (!WF::DIRECT) {  // (int4: y has x's dtype; the GGUF formats' is F32)
+      if (out_dtype == BF16) return launch_ws_o<WF, BM, BF16>(a, s);
+      if (out_dtype == F16) return launch_ws_o<WF, BM, F16>(a, s);
+    }
+    return launch_ws_o<WF, BM, F32>(a, s);
+  }
+  a.out = partials;
+  if (int rc = launch_ws_o<WF, BM, F32>(a, s)) return rc;
   return launch_splitk_reduce(partials, out, out_dtype, (int64_t)a.M * a.N, a.splits, s);
 }
 
@@ -419,6 +445,8 @@ int launch_gemm_ws_int4(const uint16_t *xb, const uint32_t *codes, const float *
   a.N = (int)N;
   a.K = (int)K;
   a.G = G;
+  a.gpr = (int)(K / G);
+  a.gsh = (G & (G - 1)) == 0 ? __builtin_ctz(G) : -1;
   a.row_bytes = K / 2;
   return launch_ws<WsInt4>(a, out_dtype, out, partials, s);
 }

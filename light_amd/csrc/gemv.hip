@@ -1205,18 +1205,48 @@ bool act_long_rows_ok(int64_t M, int64_t N, int64_t K, int dt, const void *w, co
 
 const char *matmul_q_kernel_name(int64_t M, int dt) { return use_gemm(M, dt) ? "matmul_q.gemm" : "matmul_q.gemv"; }
 
+// The workspace of one GEMM call: x as bf16, split-K partials, the bf16 copy of a weight.
+struct GemmWs {
+  uint16_t *xb, *wb;
+  float *partials;
+};
+
+static GemmWs gemm_ws_split(void *ws, int64_t M, int64_t N, int64_t K) {
+  char *base = static_cast<char *>(ws);
+  char *part = base + al256((int64_t)gemm_q4k_ws_bytes(M, K));
+  return {reinterpret_cast<uint16_t *>(base), reinterpret_cast<uint16_t *>(part + al256((int64_t)gemm_q4k_partial_bytes(M, N, K))),
+          reinterpret_cast<float *>(part)};
+}
+
+// out = xb . dequant(w)^T on bf16 x.
+static int gemm_on_bf16(const uint16_t *xb, const void *w, float *out, int64_t M, int64_t N, int64_t K, int dt, const GemmWs &g,
+                        hipStream_t s) {
+  if (dt == Q4_K) return launch_gemm_q4k_bf16(xb, w, out, g.partials, M, N, K, s);
+  if (int rc = dt == Q6_K_R ? launch_dequant_q6kr(w, g.wb, N, K, BF16, s) : launch_dequant(w, g.wb, N * K, dt, BF16, s))
+    return rc;
+  return launch_gemm_ws_bf16(xb, g.wb, out, g.partials, M, N, K, s);
+}
+
 static int run_gemm(const void *src, bool from_act, const void *w, float *out, int64_t M, int64_t N, int64_t K,
                     int dt, void *ws, hipStream_t s) {
-  char *base = static_cast<char *>(ws);
-  auto *xb = reinterpret_cast<uint16_t *>(base);
-  float *partials = reinterpret_cast<float *>(base + al256((int64_t)gemm_q4k_ws_bytes(M, K)));
-  if (int rc = launch_to_bf16(src, from_act ? kActSrc : F32, xb, M, K, s)) return rc;
-  if (dt == Q4_K) return launch_gemm_q4k_bf16(xb, w, out, partials, M, N, K, s);
-  auto *wb = reinterpret_cast<uint16_t *>(base + al256((int64_t)gemm_q4k_ws_bytes(M, K)) +
-                                          al256((int64_t)gemm_q4k_partial_bytes(M, N, K)));
-  if (int rc = dt == Q6_K_R ? launch_dequant_q6kr(w, wb, N, K, BF16, s) : launch_dequant(w, wb, N * K, dt, BF16, s))
-    return rc;
-  return launch_gemm_ws_bf16(xb, wb, out, partials, M, N, K, s);
+  const GemmWs g = gemm_ws_split(ws, M, N, K);
+  if (int rc = launch_to_bf16(src, from_act ? kActSrc : F32, g.xb, M, K, s)) return rc;
+  return gemm_on_bf16(g.xb, w, out, M, N, K, dt, g, s);
+}
+
+bool gemm_path(int64_t M, int64_t K) { return M > kGemvMaxRows && gemm_k_ok(K); }
+
+int launch_gemm_pair(const float *x, const void *w0, const void *w1, float *out0, float *out1, int64_t M, int64_t N, int64_t K,
+                     int dt, void *ws, hipStream_t s) {
+  const GemmWs g = gemm_ws_split(ws, M, N, K);
+  if (int rc = launch_to_bf16(x, F32, g.xb, M, K, s)) return rc;
+  if (int rc = gemm_on_bf16(g.xb, w0, out0, M, N, K, dt, g, s)) return rc;
+  return gemm_on_bf16(g.xb, w1, out1, M, N, K, dt, g, s);
+}
+
+int launch_gemm_on_bf16(const uint16_t *xb, const void *w, float *out, int64_t M, int64_t N, int64_t K, int dt, void *ws,
+                        hipStream_t s) {
+  return gemm_on_bf16(xb, w, out, M, N, K, dt, gemm_ws_split(ws, M, N, K), s);
 }
 
 int launch_matmul_act(const void *act, const void *w, float *out, int64_t M, int64_t N, int64_t K, int dt, void *ws,

@@ -2468,12 +2468,35 @@ int launch_int4_halves(const void *x, int x_dtype, const uint32_t *codes, const 
 // Gated projection and the MLP
 // ---------------------------------------------------------------------------
 
-// Unfused gated epilogue: out = act(g) * u, elementwise (the path for layouts the fused
-// kernel does not take).
+// Unfused gated epilogue: out = act(g) * u, elementwise (the path for layouts the fused kernel does
+// not take), as F32 or rounded to bf16 for the GEMM that follows.  Bound by memory; four outputs
+// per thread (512 x 14336, F32 -> F32, one per thread: 22.4 us, 4 TB/s).
+template <int ODT>
 __global__ __launch_bounds__(256) void gated_epilogue_kernel(const float *__restrict__ g, const float *__restrict__ u,
-                                                             float *__restrict__ out, int64_t n, int act) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) out[i] = gate_act(g[i], act) * u[i];
+                                                             void *__restrict__ out, int64_t n, int act) {
+  const int64_t i = 4 * ((int64_t)blockIdx.x * blockDim.x + threadIdx.x);
+  if (i + 4 <= n) {
+    const float4 a = *reinterpret_cast<const float4 *>(g + i), b = *reinterpret_cast<const float4 *>(u + i);
+    const float y[4] = {gate_act(a.x, act) * b.x, gate_act(a.y, act) * b.y, gate_act(a.z, act) * b.z,
+                        gate_act(a.w, act) * b.w};
+    if constexpr (ODT == F32) {
+      // (the caller's out may be 4-byte aligned only)
+#pragma unroll
+      for (int j = 0; j < 4; j++) static_cast<float *>(out)[i + j] = y[j];
+    } else {
+      *reinterpret_cast<uint2 *>(static_cast<uint16_t *>(out) + i) =
+          make_uint2((uint32_t)f2bf_rne(y[0]) | (uint32_t)f2bf_rne(y[1]) << 16,
+                     (uint32_t)f2bf_rne(y[2]) | (uint32_t)f2bf_rne(y[3]) << 16);
+    }
+    return;
+  }
+  for (int64_t e = i; e < n; e++) store_out<ODT>(out, e, gate_act(g[e], act) * u[e]);
+}
+
+template <int ODT>
+static int launch_gated_epilogue(const float *g, const float *u, void *out, int64_t n, int act, hipStream_t s) {
+  gated_epilogue_kernel<ODT><<<(unsigned)cdiv(cdiv(n, 4), 256), 256, 0, s>>>(g, u, out, n, act);
+  return check_launch("gated_epilogue");
 }
 
 static int64_t al256(int64_t b) { return (b + 255) & ~(int64_t)255; }
@@ -2501,10 +2524,13 @@ int launch_matmul_q_gated(const float *x, const void *wg, const void *wu, float 
   float *g = static_cast<float *>(ws);
   float *u = reinterpret_cast<float *>(static_cast<char *>(ws) + al256(4 * M * N));
   void *inner = static_cast<char *>(ws) + 2 * al256(4 * M * N);
-  if (int rc = launch_matmul_q(x, wg, g, M, N, K, dt, inner, s)) return rc;
-  if (int rc = launch_matmul_q(x, wu, u, M, N, K, dt, inner, s)) return rc;
-  gated_epilogue_kernel<<<(unsigned)cdiv(M * N, 256), 256, 0, s>>>(g, u, out, M * N, act);
-  return check_launch("gated_epilogue");
+  if (gemm_path(M, K)) {  // one conversion of x for both
+    if (int rc = launch_gemm_pair(x, wg, wu, g, u, M, N, K, dt, inner, s)) return rc;
+  } else {
+    if (int rc = launch_matmul_q(x, wg, g, M, N, K, dt, inner, s)) return rc;
+    if (int rc = launch_matmul_q(x, wu, u, M, N, K, dt, inner, s)) return rc;
+  }
+  return launch_gated_epilogue<F32>(g, u, out, M * N, act, s);
 }
 
 // The two-launch MLP applies: Q4_K / Q5_K, M <= 8, aligned, I a multiple of 256 (the down
@@ -2522,7 +2548,10 @@ size_t mlp_q_ws_bytes(int64_t M, int64_t H, int64_t I, int dt) {
   const size_t fused = (size_t)act_bytes(M, I);
   const size_t unfused =
       (size_t)al256(4 * M * I) + std::max(matmul_q_gated_ws_bytes(M, I, H, dt), matmul_q_ws_bytes(M, H, I, dt));
-  return std::max(fused, unfused);
+  // The GEMM chain: h as bf16, then (g, u, the pair's scratch) or the down projection's.
+  const size_t gemms = !gemm_path(M, H) || !gemm_path(M, I) ? 0
+                       : (size_t)al256(2 * M * I) + std::max(matmul_q_gated_ws_bytes(M, I, H, dt), matmul_q_ws_bytes(M, H, I, dt));
+  return std::max(std::max(fused, unfused), gemms);
 }
 
 size_t matmul_q_gated_act_ws_bytes(int64_t M, int64_t N, int64_t K, int dt) {
@@ -2707,6 +2736,18 @@ int launch_mlp_q(const float *x, const void *wg, const void *wu, const void *wd,
     // Launch 2: down projection on the prepared h.
     if (skinny_ok(M, H, I, dt, wd, hact)) return launch_skinny_act(hact, true, wd, out, M, H, I, dt, rest, s);
     return launch_gemv_q4kx_act(hact, wd, out, M, H, I, dt, s);
+  }
+  if (M > kSkinnyMaxRows || !skinny_ok(M, I, H, dt, wg, x)) {
+    if (gemm_path(M, H) && gemm_path(M, I)) {
+      // GEMMs: one conversion of x, and h rounded to bf16 by the epilogue itself (the values an F32
+      // h converted by the down projection would have; 512 x 4096 x 14336, Q4_K: 263 -> 244 us).
+      auto *hb = static_cast<uint16_t *>(ws);
+      char *rest = static_cast<char *>(ws) + al256(2 * M * I);
+      float *g = reinterpret_cast<float *>(rest), *u = reinterpret_cast<float *>(rest + al256(4 * M * I));
+      if (int rc = launch_gemm_pair(x, wg, wu, g, u, M, I, H, dt, rest + 2 * al256(4 * M * I), s)) return rc;
+      if (int rc = launch_gated_epilogue<BF16>(g, u, hb, M * I, act, s)) return rc;
+      return launch_gemm_on_bf16(hb, wd, out, M, H, I, dt, rest, s);
+    }
   }
   float *h = static_cast<float *>(ws);
   void *inner = static_cast<char *>(ws) + al256(4 * M * I);

@@ -54,6 +54,13 @@ size_t matmul_act_ws_bytes(int64_t M, int64_t N, int64_t K, int dt);
 bool matmul_act_ws_optional(int64_t M, int64_t K, int dt);
 int launch_matmul_q(const float *x, const void *w, float *out, int64_t M, int64_t N, int64_t K, int dt, void *ws,
                     hipStream_t s);
+// The many-row GEMMs (M > 8, K % 64 == 0) on shared bf16 x: two weights on one conversion of x, and
+// one weight on x already in bf16 (ws as hq_matmul_q's for that shape).
+bool gemm_path(int64_t M, int64_t K);
+int launch_gemm_pair(const float *x, const void *w0, const void *w1, float *out0, float *out1, int64_t M, int64_t N, int64_t K,
+                     int dt, void *ws, hipStream_t s);
+int launch_gemm_on_bf16(const uint16_t *xb, const void *w, float *out, int64_t M, int64_t N, int64_t K, int dt, void *ws,
+                        hipStream_t s);
 const char *matmul_q_kernel_name(int64_t M, int dt);
 // GEMV / GEMM on prepared (planar q8_1) activations.
 int launch_gemv_act(const void *act, const void *w, float *out, int64_t M, int64_t N, int64_t K, int dt,

@@ -111,7 +111,7 @@ size_t hq_matmul_q_ws_bytes(int64_t M, int64_t N, int64_t K, int w_dtype);
  * w_dtype: one of the six GGUF formats Light fuses: HQ_Q4_0, HQ_Q5_0, HQ_Q8_0, HQ_Q4_K,
  * HQ_Q5_K or HQ_Q6_K, or HQ_Q6_K_R (a Q6_K weight after hq_repack_q6k).  K must be a
  * multiple of the block size.
- *  - 3 <= M <= 16, Q4_K / Q5_K (from about 10M weights at M <= 8): f16 MFMA on exact integer weights,
+ *  - 3 <= M <= 64, Q4_K / Q5_K (from about 10M weights at M <= 8): f16 MFMA on exact integer weights,
  *    x as one or two f16 parts under a power-of-two scale per row and 256 elements.
  *  - Other M <= 8, Q4_K / Q5_K / Q6_K_R: the persistent int8-dot GEMV, x quantized to q8_1 inside its
  *    workgroups (K > 8192: into ws first).

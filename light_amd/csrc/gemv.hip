@@ -1170,7 +1170,7 @@ static size_t gemm_ws(int64_t M, int64_t N, int64_t K, int dt) {
 
 size_t matmul_q_ws_bytes(int64_t M, int64_t N, int64_t K, int dt) {
   if (M <= 0 || K <= 0 || K % 32) return 0;
-  const size_t sk = dt == Q4_K || dt == Q5_K ? skinny_ws_bytes(M, K, false) : 0;
+  const size_t sk = dt == Q4_K || dt == Q5_K ? std::max(skinny_ws_bytes(M, K, false), skinny_mid_ws_bytes(M, N, K)) : 0;
   if (use_gemm(M, dt) && gemm_k_ok(K)) return std::max(sk, gemm_ws(M, N, K, dt));
   // Long Q4_K / Q5_K rows: x quantized once, then the second K half's outputs.
   if ((dt == Q4_K || dt == Q5_K) && K > 32768 && K <= 65536 && K % 256 == 0)
@@ -1263,6 +1263,7 @@ int launch_matmul_act(const void *act, const void *w, float *out, int64_t M, int
 
 int launch_matmul_q(const float *x, const void *w, float *out, int64_t M, int64_t N, int64_t K, int dt, void *ws,
                     hipStream_t s) {
+  if (skinny_mid_ok(M, N, K, dt, w, x)) return launch_skinny_mid(x, w, out, M, N, K, dt, ws, s);
   if (skinny_ok(M, N, K, dt, w, x)) return launch_skinny(x, w, nullptr, out, M, N, K, 0, dt, ws, s);
   if (use_gemm(M, dt) && gemm_k_ok(K)) return run_gemm(x, false, w, out, M, N, K, dt, ws, s);
   if (dt == Q6_K_R) {

@@ -2524,7 +2524,7 @@ int launch_matmul_q_gated(const float *x, const void *wg, const void *wu, float 
   float *g = static_cast<float *>(ws);
   float *u = reinterpret_cast<float *>(static_cast<char *>(ws) + al256(4 * M * N));
   void *inner = static_cast<char *>(ws) + 2 * al256(4 * M * N);
-  if (gemm_path(M, K)) {  // one conversion of x for both
+  if (gemm_path(M, K) && !skinny_mid_ok(M, N, K, dt, wg, x)) {  // one conversion of x for both
     if (int rc = launch_gemm_pair(x, wg, wu, g, u, M, N, K, dt, inner, s)) return rc;
   } else {
     if (int rc = launch_matmul_q(x, wg, g, M, N, K, dt, inner, s)) return rc;
@@ -2737,7 +2737,7 @@ int launch_mlp_q(const float *x, const void *wg, const void *wu, const void *wd,
     if (skinny_ok(M, H, I, dt, wd, hact)) return launch_skinny_act(hact, true, wd, out, M, H, I, dt, rest, s);
     return launch_gemv_q4kx_act(hact, wd, out, M, H, I, dt, s);
   }
-  if (M > kSkinnyMaxRows || !skinny_ok(M, I, H, dt, wg, x)) {
+  if (!skinny_ok(M, I, H, dt, wg, x) && !skinny_mid_ok(M, I, H, dt, wg, x)) {
     if (gemm_path(M, H) && gemm_path(M, I)) {
       // GEMMs: one conversion of x, and h rounded to bf16 by the epilogue itself (the values an F32
       // h converted by the down projection would have; 512 x 4096 x 14336, Q4_K: 263 -> 244 us).

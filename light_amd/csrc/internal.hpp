@@ -119,6 +119,11 @@ int launch_skinny(const float *x, const void *w0, const void *w1, float *out, in
                   int dt, void *ws, hipStream_t s);
 int launch_skinny_act(const void *x, bool prepared, const void *w, float *out, int64_t M, int64_t N, int64_t K, int dt,
                       void *ws, hipStream_t s);
+// 17 to 64 rows (ws: skinny_mid_ws_bytes).
+bool skinny_mid_ok(int64_t M, int64_t N, int64_t K, int dt, const void *w, const void *x);
+size_t skinny_mid_ws_bytes(int64_t M, int64_t N, int64_t K);
+int launch_skinny_mid(const float *x, const void *w, float *out, int64_t M, int64_t N, int64_t K, int dt, void *ws,
+                      hipStream_t s);
 int launch_skinny_int4(const void *x, int x_dtype, const uint32_t *codes, const float *sc, const float *zr, void *y,
                        int64_t M, int64_t N, int64_t K, int G, void *ws, hipStream_t s);
 // The Q4_K / Q5_K halves for M >= 2 rows of F32 x: one launch per half for every row of x.

@@ -1,5 +1,5 @@
-// skinny.hip -- quantized-weight product for a few rows of x (3 <= M <= 16) on MFMA (gfx950):
-// Q4_K, Q5_K and int4 (group a multiple of 128), plain or gated (SwiGLU / GELU-erf).
+// skinny.hip -- quantized-weight product for a few rows of x on MFMA (gfx950): 3 <= M <= 16, Q4_K, Q5_K
+// and int4 (group a multiple of 128), plain or gated (SwiGLU / GELU-erf); 17 <= M <= 64, Q4_K and Q5_K.
 //
 // Role: Light's matmul_q and int4_gemv for small batches (ops/matmul_q.go:61-75,
 // ops/int4.go:87-99) and its gated MLP projection (models/llama.go:1306-1328): a decode batch or
@@ -32,6 +32,7 @@
 #include "dma.hpp"
 #include "internal.hpp"
 
+#include <algorithm>
 #include <atomic>
 
 namespace hq {
@@ -46,6 +47,7 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kXDup = 0, kXPair = 1, kX16 = 2;  // how the sixteen A rows hold x
+constexpr int kX64 = 3;                         // records of up to 64 rows (skinny_mid_kernel)
 
 constexpr uint32_t K1024 = 0x64006400u;  // f16 pair (1024, 1024)
 
@@ -209,7 +211,7 @@ struct SkI4 {
 // ---- x: rows of a unit in A fragment order ----------------------------------------------
 // Record of one unit for P rows: fragments [ST][4][P] x 16 B, then (K formats) sub-block sums
 // [4][P] x 8 B = (hi 2g, hi 2g+1, lo 2g, lo 2g+1), then by A row xs f32 [16] (the row's power of
-// two) and (int4) sx f32 [16] (the unit's sum).  In memory P is M (kXPair: 2 M), so that a CU
+// two; kX64: [64]) and (int4) sx f32 [16] (the unit's sum).  In memory P is M (kXPair: 2 M), so that a CU
 // fetches no padding (every CU reads all of x from L2); in LDS the A rows, 8 or 16.
 template <class F, int XM>
 struct XRec {
@@ -217,7 +219,7 @@ struct XRec {
   __host__ __device__ static constexpr int rows(int M) { return XM == kXPair ? 2 * M : M; }
   __host__ __device__ static constexpr int mins(int P) { return F::ST * 4 * P * 16; }
   __host__ __device__ static constexpr int xs(int P) { return mins(P) + (F::INT4 ? 0 : 32 * P); }
-  __host__ __device__ static constexpr int bytes(int P) { return xs(P) + (F::INT4 ? 128 : 64); }
+  __host__ __device__ static constexpr int bytes(int P) { return xs(P) + (XM == kX64 ? 256 : F::INT4 ? 128 : 64); }
   static constexpr int BYTES = bytes(ROWS);
 };
 
@@ -808,6 +810,116 @@ __global__ __launch_bounds__(256) void skinny_x_kernel(SkinnyArgs a, uint8_t *xf
   convert_row<F, XM>(v, m, lane, xf + (int64_t)c * (UPC * R::bytes(P)), P);
 }
 
+// ---- 17 to 64 rows ---------------------------------------------------------------------------
+// Eight tiles of 16 weight rows per workgroup, one per wave, over one of S parts of K (F32 partials,
+// added by splitk_reduce_kernel).  All waves multiply the same unit, so x's record (up to 64 rows,
+// 34 KB) is staged in LDS once per workgroup, and each unpacked weight fragment meets MT of its
+// row tiles.  Per unit: wait for this wave's direct loads, one barrier, request the next unit, work.
+// Against the bf16 GEMM of 64-row tiles, whose f32 dequantization (3.5 VALU instructions per
+// weight against 1.4 here) bounds it.
+template <class F>
+struct SkinnyMidLds {
+  static constexpr int WST = (16 * F::BB + 1023) / 1024 * 1024;  // a wave's weights of one unit
+  static constexpr int NW = WST / 1024;
+  static constexpr int XST = (XRec<F, kX64>::bytes(64) + 1023) / 1024 * 1024;
+  static constexpr int STAGE = XST + 8 * WST, BYTES = 2 * STAGE;
+  static_assert(BYTES <= 160 * 1024, "LDS");
+};
+
+template <class F, int MT>
+__global__ __launch_bounds__(512) void skinny_mid_kernel(SkinnyArgs a) {
+  using R = XRec<F, kX64>;
+  using T = SkinnyMidLds<F>;
+  constexpr int PR = F::BB / 16;  // pieces of a row's unit
+  extern __shared__ __align__(16) uint8_t smem[];
+  const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int g = lane >> 4, r = lane & 15;
+  const int S = (int)gridDim.y;
+  const int u0 = a.nun * (int)blockIdx.y / S, u1 = a.nun * ((int)blockIdx.y + 1) / S;  // u0 < u1: S <= nun
+  const int P = a.M, rec = R::bytes(P);
+  const int row0 = ((int)blockIdx.x * 8 + wave) * 16;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)smem;
+  // The record's direct loads of this wave: 1 KB each, wave + 8 k (at most five), the last shifted
+  // back to end with the record.
+  const int nx = (rec + 1023) >> 10, ndx = (nx - wave + 7) >> 3;
+  uint32_t woff[T::NW];
+#pragma unroll
+  for (int k = 0; k < T::NW; k++) {
+    int p = k * 64 + lane;
+    p = p < 16 * PR ? p : 16 * PR - 1;
+    const int row = row0 + p / PR;
+    woff[k] = (uint32_t)(row < a.N ? row : a.N - 1) * a.row_bytes + (uint32_t)(p % PR) * 16;
+  }
+  auto issue = [&](int u, int buf) __attribute__((always_inline)) {
+    u = u < u1 ? u : u1 - 1;  // (the last request repeats)
+    const uint32_t dst = lds0 + buf * T::STAGE;
+    const uint8_t *xr = a.xf + (int64_t)u * rec;
+    for (int k = 0; k < ndx; k++) {  // wave-uniform
+      const int o = (wave + 8 * k) * 1024, oc = o + 1024 <= rec ? o : rec - 1024;
+      dma16s(xr, (uint32_t)(oc + lane * 16), __builtin_amdgcn_readfirstlane(dst + oc));
+    }
+#pragma unroll
+    for (int k = 0; k < T::NW; k++)
+      dma16s(a.w0, woff[k] + (uint32_t)(u * F::BB), __builtin_amdgcn_readfirstlane(dst + T::XST + wave * T::WST + k * 1024));
+  };
+  f32x4 acc[MT];
+#pragma unroll
+  for (int m = 0; m < MT; m++) acc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
+  issue(u0, 0);
+  for (int u = u0; u < u1; u++) {
+    const int buf = (u - u0) & 1;
+    wait_vm<0>();
+    __syncthreads();  // unit u is staged; every wave is done with the other buffer
+    issue(u + 1, buf ^ 1);
+    const uint8_t *x = smem + buf * T::STAGE;
+    typename F::Raw raw;
+    F::load_lds(x + T::XST + wave * T::WST + r * F::BB, 0, PR, g, raw);
+    const typename F::Sc sc = F::decode(raw, g);
+    f32x4 q[MT], mn[MT];
+#pragma unroll
+    for (int m = 0; m < MT; m++) q[m] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const uint8_t *xa[MT];
+#pragma unroll
+    for (int m = 0; m < MT; m++) {
+      const int row = m * 16 + r;
+      xa[m] = x + (g * P + (row < P ? row : P - 1)) * 16;
+    }
+#pragma unroll
+    for (int i = 0; i < F::ST; i++) {
+      const f16x8 b = F::frag(raw, sc, g, i);
+#pragma unroll
+      for (int m = 0; m < MT; m++)
+        q[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(as_h8(*reinterpret_cast<const u32x4 *>(xa[m] + i * (64 * P))), b, q[m], 0,
+                                                       0, 0);
+    }
+#pragma unroll
+    for (int m = 0; m < MT; m++) {
+      const int row = m * 16 + r;
+      const u32x2 xm = *reinterpret_cast<const u32x2 *>(x + R::mins(P) + (g * P + (row < P ? row : P - 1)) * 8);
+      mn[m] = f32x4{0.f, 0.f, 0.f, 0.f};
+      mn[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(as_h8(u32x4{xm[0], xm[1], 0, 0}), as_h8(sc.mn), mn[m], 0, 0, 0);
+    }
+#pragma unroll
+    for (int m = 0; m < MT; m++) {
+      const f32x4 xs = *reinterpret_cast<const f32x4 *>(x + R::xs(P) + (m * 16 + 4 * g) * 4);
+#pragma unroll
+      for (int j = 0; j < 4; j++) acc[m][j] = __fmaf_rn(xs[j], __fmaf_rn(sc.d, q[m][j], -(sc.dmin * mn[m][j])), acc[m][j]);
+    }
+  }
+  wait_vm<0>();
+  float *out = static_cast<float *>(a.out) + (int64_t)blockIdx.y * a.M * a.N;
+  const int col = row0 + r;
+  if (col < a.N) {
+#pragma unroll
+    for (int m = 0; m < MT; m++)
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        const int row = m * 16 + 4 * g + j;
+        if (row < a.M) out[(int64_t)row * a.N + col] = acc[m][j];
+      }
+  }
+}
+
 // ---- host side ------------------------------------------------------------------------------
 
 namespace {
@@ -987,6 +1099,71 @@ int launch_skinny_act(const void *x, bool prepared, const void *w, float *out, i
                     : run_any<SkQk<true>, false, kXQuant, F32>(a, pair, ws, s);
   return prepared ? run_any<SkQk<false>, false, kXAct, F32>(a, pair, ws, s)
                   : run_any<SkQk<false>, false, kXQuant, F32>(a, pair, ws, s);
+}
+
+// ---- 17 <= M <= 64, Q4_K / Q5_K (skinny_mid_kernel) ----
+// K parts: the fewest rounds of workgroups (one per CU) times units per part, a part's start and its
+// share of the reduce counted as three units.
+static int mid_splits(int64_t N, int64_t K) {
+  const int64_t groups = cdiv(N, 128), nun = K / 256, cus = device_cus();
+  int64_t best = INT64_MAX, s = 1;
+  for (int64_t c = 1; c <= 16 && (c == 1 || c * 2 <= nun); c++) {
+    const int64_t cost = cdiv(groups * c, cus) * (cdiv(nun, c) + (c > 1 ? 3 : 2));
+    if (cost < best) best = cost, s = c;
+  }
+  return (int)s;
+}
+
+// Every such call (us, the bf16 GEMM with its conversion and reduce / this; Q4_K): 14336 x 4096 M = 24 28.2 /
+// 17.4, M = 40 28.7 / 22.9, M = 64 30.0 / 27.1; 4096 x 14336 M = 64 36.4 / 26.5; 512 x 1024 M = 20 13.7 / 8.9;
+// 28672 x 8192 M = 40 94.7 / 63.7.  Q5_K, which the GEMM first expands to bf16 in memory: 14336 x 4096 M = 40
+// 94.1 / 23.4.
+bool skinny_mid_ok(int64_t M, int64_t N, int64_t K, int dt, const void *w, const void *x) {
+  return (dt == Q4_K || dt == Q5_K) && M > kSkinnyMaxRows && M <= 64 && K > 0 && K % 256 == 0 && K <= kSkinnyMaxK && N >= 1 &&
+         N * (K / 256) * block_info(dt).bytes <= UINT32_MAX && ((uintptr_t)w & 15) == 0 && ((uintptr_t)x & 15) == 0;
+}
+
+static size_t mid_rec_bytes(int64_t M, int64_t K) {
+  return (size_t)((K / 256 * XRec<SkQk<false>, kX64>::bytes((int)M) + 255) & ~(int64_t)255);
+}
+
+size_t skinny_mid_ws_bytes(int64_t M, int64_t N, int64_t K) {
+  if (M <= kSkinnyMaxRows || M > 64 || N < 1 || K % 256 || K > kSkinnyMaxK) return 0;
+  const int s = mid_splits(N, K);
+  return mid_rec_bytes(M, K) + (s > 1 ? (size_t)s * M * N * 4 : 0);
+}
+
+int launch_splitk_reduce(const float *part, void *out, int out_dtype, int64_t n, int splits, hipStream_t s);
+
+template <class F, int MT>
+static int run_mid(SkinnyArgs a, float *out, void *ws, hipStream_t s) {
+  constexpr int lds = SkinnyMidLds<F>::BYTES;
+  auto *kern = &skinny_mid_kernel<F, MT>;
+  static std::atomic<bool> done[64];
+  if (int rc = allow_lds(kern, done, lds)) return rc;
+  auto *xf = static_cast<uint8_t *>(ws);
+  auto *part = reinterpret_cast<float *>(xf + mid_rec_bytes(a.M, a.K));
+  skinny_x_kernel<F, kX64, F32><<<(unsigned)cdiv((int64_t)a.nun * a.M, 4), 256, 0, s>>>(a, xf);
+  if (int rc = check_launch("skinny_x")) return rc;
+  const int S = mid_splits(a.N, a.K);
+  a.xf = xf;
+  a.out = S > 1 ? part : out;
+  kern<<<dim3((unsigned)cdiv(a.N, 128), (unsigned)S), 512, lds, s>>>(a);
+  if (int rc = check_launch("skinny_mid")) return rc;
+  return S > 1 ? launch_splitk_reduce(part, out, F32, (int64_t)a.M * a.N, S, s) : HQ_OK;
+}
+
+template <class F>
+static int run_mid_m(const SkinnyArgs &a, float *out, void *ws, hipStream_t s) {
+  if (a.M <= 32) return run_mid<F, 2>(a, out, ws, s);
+  if (a.M <= 48) return run_mid<F, 3>(a, out, ws, s);
+  return run_mid<F, 4>(a, out, ws, s);
+}
+
+int launch_skinny_mid(const float *x, const void *w, float *out, int64_t M, int64_t N, int64_t K, int dt, void *ws,
+                      hipStream_t s) {
+  const SkinnyArgs a = skinny_args(x, w, out, M, N, K, dt);
+  return dt == Q5_K ? run_mid_m<SkQk<true>>(a, out, ws, s) : run_mid_m<SkQk<false>>(a, out, ws, s);
 }
 
 int launch_skinny_int4(const void *x, int x_dtype, const uint32_t *codes, const float *sc, const float *zr, void *y,

@@ -63,6 +63,19 @@ def test_small_weights(dev, M, N, K):
 
 
 @pytest.mark.parametrize("dt", [hipq.Q4_K, hipq.Q5_K])
+@pytest.mark.parametrize("M", [17, 32, 33, 48, 49, 64])
+@pytest.mark.parametrize("N,K", [(1, 256), (130, 512), (127, 768), (2567, 4096), (4000, 14336), (40001, 1024)])
+def test_mid_rows(dev, dt, M, N, K):
+    """17 to 64 rows: row-tile, column-group and K-part remainders, one part and sixteen."""
+    print(f"[case] skinny mid dt={hipq.NAMES[dt]} M={M} N={N} K={K}", flush=True)
+    w, wd = _weight(dt, N, K, dev, seed=N + K)
+    x = _x(M, K, dev, seed=M)
+    y = hipq.matmul_q(x, w, N, K, dt)
+    assert _err(y, x.double() @ wd.t(), x, wd) <= 2.5e-4
+    assert torch.equal(y, hipq.matmul_q(x, w, N, K, dt)), "not deterministic"
+
+
+@pytest.mark.parametrize("dt", [hipq.Q4_K, hipq.Q5_K])
 @pytest.mark.parametrize("M,N,K", [(3, 2567, 4096), (8, 5008, 2048), (16, 1000, 3840), (5, 1608, 6400), (12, 6000, 4352)])
 def test_gated(dev, dt, M, N, K):
     print(f"[case] skinny gated dt={hipq.NAMES[dt]} M={M} N={N} K={K}", flush=True)

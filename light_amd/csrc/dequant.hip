@@ -16,6 +16,16 @@
 
 namespace hq {
 
+// Two f32 -> packed bf16 by the hardware's conversion, equal to f2bf_rne for all 2^32 inputs (checked,
+// NaNs included) at one instruction instead of about eight per value.
+__device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  const bf16x2 v = {(__bf16)a, (__bf16)b};
+  uint32_t u;
+  __builtin_memcpy(&u, &v, 4);
+  return u;
+}
+
 template <int DT, int ODT>
 __global__ __launch_bounds__(256) void dequant_kernel(const uint8_t *__restrict__ w, void *__restrict__ out,
                                                       int64_t n8) {
@@ -29,10 +39,10 @@ __global__ __launch_bounds__(256) void dequant_kernel(const uint8_t *__restrict_
     o[1] = make_float4(y[4], y[5], y[6], y[7]);
   } else {
     uint4 v;
-    v.x = f2bf_rne(y[0]) | (uint32_t)f2bf_rne(y[1]) << 16;
-    v.y = f2bf_rne(y[2]) | (uint32_t)f2bf_rne(y[3]) << 16;
-    v.z = f2bf_rne(y[4]) | (uint32_t)f2bf_rne(y[5]) << 16;
-    v.w = f2bf_rne(y[6]) | (uint32_t)f2bf_rne(y[7]) << 16;
+    v.x = pack_bf16(y[0], y[1]);
+    v.y = pack_bf16(y[2], y[3]);
+    v.z = pack_bf16(y[4], y[5]);
+    v.w = pack_bf16(y[6], y[7]);
     *reinterpret_cast<uint4 *>(static_cast<uint16_t *>(out) + t * 8) = v;
   }
 }

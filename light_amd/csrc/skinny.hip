@@ -29,6 +29,7 @@
 //  * Weights reach LDS by direct loads of whole row runs.  (The MFMA operand order -- lane l reads
 //    row l % 16 -- as plain loads touches a cache line per lane: 33 MB in 9.4 us against 6.9 us.)
 #include "actq.hpp"
+#include "decode.hpp"
 #include "dma.hpp"
 #include "internal.hpp"
 
@@ -92,6 +93,7 @@ struct SkinnyArgs {
   const float *s, *z;      // int4 scales / zeros (N, K / G)
   void *out;               // (M, N)
   int M, N, K, nun, tiles, act;
+  int xdt;                 // x's dtype (F32, BF16, F16; kXAct)
   int gpr, gunits;         // int4: groups per row, units per group
   uint32_t row_bytes, last;  // last: N row_bytes - 16
   // skinny_kernel's plan: groups of 256 k per chunk, chunks, pieces of a staged row, tile sets.
@@ -109,6 +111,7 @@ namespace {
 template <bool Q5>
 struct SkQk {
   static constexpr bool INT4 = false;
+  static constexpr int DT = Q5 ? Q5_K : Q4_K;
   static constexpr int KU = 256, ST = 8, BB = Q5 ? 176 : 144, QO = Q5 ? 48 : 16;
   struct Raw {
     u32x4 hd, q0, q1, h0, h1;  // h0, h1: Q5_K's fifth bits
@@ -404,6 +407,54 @@ __device__ __forceinline__ void unit_mma(const typename F::Raw &w, const XFrag<F
   }
 }
 
+// Output (m, n) over the columns [k0, k1) of w, from its f16 form y.  That form splits a weight into
+// sc * q and a minimum (int4: q and z), so an infinite x meets them as Inf - Inf.  A y that is not
+// finite is therefore worked out again as f32 arithmetic has it: x's non-finite elements times their
+// weights (the finite ones add nothing to those); without such an element y stands.  One compare per
+// output otherwise.
+template <class F>
+__device__ __forceinline__ float settle(const SkinnyArgs &a, const uint8_t *w, int m, int n, int k0, int k1, float y) {
+  if (__builtin_expect(__builtin_isfinite(y) || a.xdt < 0, 1)) return y;
+  float s = 0.f;
+  bool any = false;
+#pragma unroll 1
+  for (int k = k0; k < k1 && s == s; k += 8) {  // (NaN stays NaN)
+    const int64_t i = (int64_t)m * a.K + k;
+    float v[8];
+    if (a.xdt == F32) {
+      const f32x4 *p = reinterpret_cast<const f32x4 *>(static_cast<const float *>(a.x) + i);
+      const f32x4 p0 = p[0], p1 = p[1];
+#pragma unroll
+      for (int j = 0; j < 8; j++) v[j] = j < 4 ? p0[j] : p1[j - 4];
+    } else {
+      const u32x4 p = *reinterpret_cast<const u32x4 *>(static_cast<const uint16_t *>(a.x) + i);
+#pragma unroll
+      for (int j = 0; j < 8; j++) {
+        const uint32_t h = (j & 1) ? p[j >> 1] >> 16 : p[j >> 1] & 0xffffu;
+        v[j] = a.xdt == BF16 ? bf2f(h) : h2f(h);
+      }
+    }
+    bool bad = false;
+#pragma unroll
+    for (int j = 0; j < 8; j++) bad |= !__builtin_isfinite(v[j]);
+    if (!bad) continue;
+    any = true;
+    float d[8];
+    if constexpr (F::INT4) {
+      const int64_t gi = (int64_t)n * a.gpr + k / (128 * a.gunits);
+      const uint32_t q = reinterpret_cast<const uint32_t *>(w + (int64_t)n * a.row_bytes)[k >> 3];
+#pragma unroll
+      for (int j = 0; j < 8; j++) d[j] = a.s[gi] * ((float)((q >> (4 * j)) & 15) - a.z[gi]);
+    } else {
+      decode8<F::DT>(w + (int64_t)n * a.row_bytes, k >> 3, d);
+    }
+#pragma unroll
+    for (int j = 0; j < 8; j++)
+      if (!__builtin_isfinite(v[j])) s += v[j] * d[j];
+  }
+  return any ? s : y;
+}
+
 template <int ODT>
 __device__ __forceinline__ void store_y(void *out, int64_t i, float y) {
   if constexpr (ODT == F32)
@@ -605,9 +656,11 @@ __global__ __launch_bounds__(1024) void skinny_kernel(SkinnyArgs a) {
       const int c = o & 15, m = (o >> 4) & (XROWS - 1), q = (o >> 4) / XROWS;
       float y = sum_parts<KW, XM>(pb + q * KW * 256, c, m);
       const int col = row0 + q * 16 + c;
+      if (m >= a.M || col >= a.N) continue;
+      if constexpr (XDT >= 0) y = settle<F>(a, GATED && j ? a.w1 : a.w0, m, col, 0, a.K, y);
       if (GATED && j == 0) {
         gs[k] = y;
-      } else if (m < a.M && col < a.N) {
+      } else {
         if constexpr (GATED) y = gate_act(gs[k], a.act) * y;
         store_y<ODT>(a.out, (int64_t)m * a.N + col, y);
       }
@@ -780,12 +833,14 @@ __global__ __launch_bounds__(1024) void skinny_long_kernel(SkinnyArgs a) {
     __syncthreads();
     if (t < 16 * XROWS) {
       const int c = t & 15, m = t >> 4, col = row0_of(k / NW) + c;
-      float y = sum_parts<CW, XM>(part, c, m);
-      if (GATED && k % NW == 0) {
-        gs = y;
-      } else if (m < a.M && col < a.N) {
-        if constexpr (GATED) y = gate_act(gs, a.act) * y;
-        store_y<ODT>(a.out, (int64_t)m * a.N + col, y);
+      if (m < a.M && col < a.N) {
+        float y = settle<F>(a, k % NW ? a.w1 : a.w0, m, col, 0, a.K, sum_parts<CW, XM>(part, c, m));
+        if (GATED && k % NW == 0) {
+          gs = y;
+        } else {
+          if constexpr (GATED) y = gate_act(gs, a.act) * y;
+          store_y<ODT>(a.out, (int64_t)m * a.N + col, y);
+        }
       }
     }
   }
@@ -915,7 +970,7 @@ __global__ __launch_bounds__(512) void skinny_mid_kernel(SkinnyArgs a) {
 #pragma unroll
       for (int j = 0; j < 4; j++) {
         const int row = m * 16 + 4 * g + j;
-        if (row < a.M) out[(int64_t)row * a.N + col] = acc[m][j];
+        if (row < a.M) out[(int64_t)row * a.N + col] = settle<F>(a, a.w0, row, col, u0 * 256, u1 * 256, acc[m][j]);
       }
   }
 }
@@ -1083,6 +1138,7 @@ int launch_skinny(const float *x, const void *w0, const void *w1, float *out, in
   SkinnyArgs a = skinny_args(x, w0, out, M, N, K, dt);
   a.w1 = static_cast<const uint8_t *>(w1);
   a.act = act;
+  a.xdt = F32;
   const bool pair = skinny_pair(K);
   if (dt == Q5_K)
     return w1 ? run_any<SkQk<true>, true, F32, F32>(a, pair, ws, s) : run_any<SkQk<true>, false, F32, F32>(a, pair, ws, s);
@@ -1092,7 +1148,8 @@ int launch_skinny(const float *x, const void *w0, const void *w1, float *out, in
 // x as prepared activations, or F32 x taken through their quantization (the same results); M <= 8.
 int launch_skinny_act(const void *x, bool prepared, const void *w, float *out, int64_t M, int64_t N, int64_t K, int dt,
                       void *ws, hipStream_t s) {
-  const SkinnyArgs a = skinny_args(x, w, out, M, N, K, dt);
+  SkinnyArgs a = skinny_args(x, w, out, M, N, K, dt);
+  a.xdt = kXAct;
   const bool pair = skinny_pair(K);
   if (dt == Q5_K)
     return prepared ? run_any<SkQk<true>, false, kXAct, F32>(a, pair, ws, s)
@@ -1162,7 +1219,8 @@ static int run_mid_m(const SkinnyArgs &a, float *out, void *ws, hipStream_t s) {
 
 int launch_skinny_mid(const float *x, const void *w, float *out, int64_t M, int64_t N, int64_t K, int dt, void *ws,
                       hipStream_t s) {
-  const SkinnyArgs a = skinny_args(x, w, out, M, N, K, dt);
+  SkinnyArgs a = skinny_args(x, w, out, M, N, K, dt);
+  a.xdt = F32;
   return dt == Q5_K ? run_mid_m<SkQk<true>>(a, out, ws, s) : run_mid_m<SkQk<false>>(a, out, ws, s);
 }
 
@@ -1170,6 +1228,7 @@ int launch_skinny_int4(const void *x, int x_dtype, const uint32_t *codes, const 
                        int64_t M, int64_t N, int64_t K, int G, void *ws, hipStream_t s) {
   SkinnyArgs a = {};
   a.x = x;
+  a.xdt = x_dtype;
   a.w0 = reinterpret_cast<const uint8_t *>(codes);
   a.s = sc;
   a.z = zr;

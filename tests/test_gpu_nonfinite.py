@@ -63,3 +63,61 @@ def test_int4_nonfinite_row(dev, M, xdt):
     ok = hipq.int4_matmul(x.to(xdt), codes, s, z, G)
     x[0, 100] = float("nan")
     _rows_check(hipq.int4_matmul(x.to(xdt), codes, s, z, G), ok)
+
+
+def _same_class(y, want):
+    """Every output is NaN, +Inf or -Inf where float64 on the dequantized weight has it so."""
+    want = want.to(torch.float32)
+    assert torch.equal(torch.isnan(y), torch.isnan(want))
+    inf = torch.isinf(want)
+    assert torch.equal(torch.isinf(y), inf) and torch.equal(torch.sign(y[inf]), torch.sign(want[inf]))
+
+
+def _plant(x):
+    """Row 0: one Inf; row 1: two of one sign far apart; row 2: Inf and -Inf; the last: a NaN beside an Inf
+    (with three rows, the last is row 2)."""
+    K, x = x.shape[1], x.clone()
+    x[0, 37] = float("-inf")
+    x[1, 5], x[1, K - 3] = float("inf"), float("inf")
+    x[2, K // 2], x[2, K // 2 + 9] = float("inf"), float("-inf")
+    x[-1, K - 1], x[-1, 0] = float("nan"), float("inf")
+    return x
+
+
+# 3 to 8 rows from 10M weights (one part of x, two), 9 to 16 and 17 to 64 (one K part, several): rows of up
+# to 4096 and longer ones of skinny.hip, with a ragged N.
+@pytest.mark.parametrize("dt", [hipq.Q4_K, hipq.Q5_K])
+@pytest.mark.parametrize("M,N,K", [(3, 2567, 4096), (5, 5008, 2048), (8, 1601, 6656), (4, 1601, 16640), (9, 97, 2048),
+                                   (16, 97, 5120), (17, 97, 2304), (40, 130, 4096), (64, 40001, 512)])
+def test_infinities_as_in_f32(dev, dt, M, N, K):
+    print(f"[case] infinities dt={hipq.NAMES[dt]} M={M} N={N} K={K}", flush=True)
+    w = torch.from_numpy(synth.gguf_weight(dt, N, K, synth.rng(K + M))).to(dev)
+    wd = hipq.dequant(w, N * K, dt).view(N, K).double()
+    x = torch.randn(M, K, device=dev)
+    ok = hipq.matmul_q(x, w, N, K, dt)
+    x = _plant(x)
+    y = hipq.matmul_q(x, w, N, K, dt)
+    _same_class(y, x.double() @ wd.t())
+    if M > 4:
+        assert torch.equal(y[3:-1], ok[3:-1]), "other rows changed"
+    if 4 < M <= 16 or K == 4096:  # (other gated calls of up to four rows quantize x to int8)
+        h = hipq.matmul_q_gated(x, w, w, N, K, dt)
+        a = x.double() @ wd.t()
+        _same_class(h, torch.nn.functional.silu(a) * a)
+
+
+@pytest.mark.parametrize("xdt", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,N,K", [(3, 3208, 4096), (8, 5000, 2688), (5, 2056, 18944), (9, 12296, 4096), (16, 4104, 8192)])
+def test_int4_infinities_as_in_f32(dev, xdt, M, N, K):
+    print(f"[case] infinities int4 x={xdt} M={M} N={N} K={K}", flush=True)
+    codes, s, z = (torch.from_numpy(a).to(dev) for a in synth.int4_weight(N, K, 128, synth.rng(N)))
+    codes, z = codes.view(torch.int32), z.round()  # (whole zeros: weights of exactly 0 come up)
+    wd = hipq.int4_dequant(codes, s, z, 128).double()
+    x = torch.randn(M, K, device=dev).to(xdt)
+    ok = hipq.int4_matmul(x, codes, s, z, 128)
+    x = _plant(x)
+    y = hipq.int4_matmul(x, codes, s, z, 128)
+    assert (wd == 0).any()
+    _same_class(y.float(), x.double() @ wd.t())
+    if M > 4:
+        assert torch.equal(y[3:-1], ok[3:-1]), "other rows changed"

@@ -179,10 +179,10 @@ int hq_matmul_q_gated_act(const float *x, const void *wg, const void *wu, void *
 /* The gated MLP block of a decoder layer:
  *   out (M, H) F32 = (act(x @ dequant(wg)^T) * (x @ dequant(wu)^T)) @ dequant(wd)^T
  * with x (M, H) F32, wg and wu (I, H), wd (H, I), all of w_dtype; act as above.
- * For Q4_K with M <= 8 this is hq_matmul_q_gated_act followed by hq_matmul_q_act, bit for bit: at
- * M <= 2 (and for small weights) two launches, the gated gate/up GEMV, which writes its output
- * already quantized for the next matmul into ws, and the down GEMV on it.  Other cases run
- * hq_matmul_q_gated into ws and then hq_matmul_q.
+ * For Q4_K / Q5_K with M <= 8 where both halves take the int8 GEMV (M <= 2, and small weights) this
+ * is two launches, hq_matmul_q_gated_act (the gated gate/up GEMV, which writes its output already
+ * quantized for the next matmul into ws) and hq_matmul_q_act (the down GEMV on it), bit for bit.
+ * Other cases run hq_matmul_q_gated into ws and then hq_matmul_q, bit for bit.
  * Light: models/llama.go:1306-1333 (GatedLinear or MatMulQ/SiLU/Mul, then DownProj).
  * No counterpart op in Light. */
 size_t hq_mlp_q_ws_bytes(int64_t M, int64_t H, int64_t I, int w_dtype);
@@ -206,9 +206,8 @@ int hq_mlp_q(const float *x, const void *wg, const void *wu, const void *wd, flo
  * GEMVs use both levels.  The layout is internal and may change with the version. */
 size_t hq_act_bytes(int64_t M, int64_t K);
 int hq_quantize_act(const void *x, int x_dtype, void *act, int64_t M, int64_t K, hq_stream_t stream);
-/* Workspace hq_matmul_q_act uses beyond the act buffer.  For Q4_K / Q5_K at 3 <= M <= 8 with rows
- * past 4096 it is optional: without it (a smaller ws, or a library workspace that cannot grow
- * during capture) the int8 GEMV serves the call. */
+/* Workspace hq_matmul_q_act needs beyond the act buffer (0 for M <= 8, except rows that run as K
+ * parts). */
 size_t hq_matmul_q_act_ws_bytes(int64_t M, int64_t N, int64_t K, int w_dtype);
 /* out (M, N) F32 = x @ dequant(w)^T from prepared activations.  For M <= 8, and for
  * any M when K is not a multiple of 64, the weight must take the int8 GEMV (16-byte

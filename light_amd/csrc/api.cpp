@@ -503,14 +503,10 @@ int hq_matmul_q_act(const void *act, const void *w, float *out, int64_t M, int64
     return fail(HQ_EUNSUPPORTED, call, "weight layout needs the F32 path (hq_matmul_q)");
   hipStream_t s = resolve(stream);
   size_t need = hq_matmul_q_act_ws_bytes(M, N, K, w_dtype);
-  const bool optional = matmul_act_ws_optional(M, K, w_dtype);
   if (need && !ws) {
-    const int rc = workspace(need, s, &ws, call);
-    if (rc && !optional) return rc;
-    if (rc) ws = nullptr;
+    if (int rc = workspace(need, s, &ws, call)) return rc;
   } else if (need && ws_bytes < need) {
-    ws = nullptr;
-    if (!optional) return fail(HQ_ENOMEM, call, "workspace %zu bytes < %zu needed", ws_bytes, need);
+    return fail(HQ_ENOMEM, call, "workspace %zu bytes < %zu needed", ws_bytes, need);
   }
   TraceSpan span(matmul_q_kernel_name(M, w_dtype), s);
   return launch_matmul_act(act, w, out, M, N, K, w_dtype, ws, s);

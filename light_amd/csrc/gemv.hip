@@ -1190,12 +1190,7 @@ static bool long_rows_dt(int64_t K, int dt) {
 size_t matmul_act_ws_bytes(int64_t M, int64_t N, int64_t K, int dt) {
   if (M <= 0 || K <= 0 || K % 32) return 0;
   if (use_gemm(M, dt) && gemm_k_ok(K)) return gemm_ws(M, N, K, dt);
-  if (long_rows_dt(K, dt)) return N > 0 ? (size_t)(4 * M * N) : 0;
-  return dt == Q4_K || dt == Q5_K ? skinny_ws_bytes(M, K, false) : 0;
-}
-
-bool matmul_act_ws_optional(int64_t M, int64_t K, int dt) {
-  return !(use_gemm(M, dt) && gemm_k_ok(K)) && !long_rows_dt(K, dt);
+  return long_rows_dt(K, dt) && N > 0 ? (size_t)(4 * M * N) : 0;
 }
 
 bool act_long_rows_ok(int64_t M, int64_t N, int64_t K, int dt, const void *w, const void *act) {
@@ -1256,8 +1251,9 @@ int launch_matmul_act(const void *act, const void *w, float *out, int64_t M, int
     return launch_staged_parts(act, w, out, static_cast<float *>(ws), M, N, K, dt, s);
   if (q4kx_halves_ok(M, N, K, dt, w, act))
     return launch_gemv_q4kx_act_halves(act, w, out, static_cast<float *>(ws), M, N, K, dt, s);
-  if (M <= kGemvMaxRows && skinny_ok(M, N, K, dt, w, act) && (ws || skinny_ws_bytes(M, K, false) == 0))
-    return launch_skinny_act(act, true, w, out, M, N, K, dt, ws, s);
+  // (Longer rows would need a workspace for x's records, which this call has none for: the GEMV.)
+  if (M <= kGemvMaxRows && skinny_ws_bytes(M, K, false) == 0 && skinny_ok(M, N, K, dt, w, act))
+    return launch_skinny_act(act, w, out, M, N, K, dt, s);
   return launch_gemv_act(act, w, out, M, N, K, dt, s);
 }
 

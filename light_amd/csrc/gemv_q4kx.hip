@@ -2718,24 +2718,14 @@ int launch_matmul_q_gated_act(const float *x, const void *wg, const void *wu, ui
 
 int launch_mlp_q(const float *x, const void *wg, const void *wu, const void *wd, float *out, int64_t M, int64_t H,
                  int64_t I, int dt, int act, void *ws, hipStream_t s) {
-  if (mlp_fused_ok(M, H, I, dt, wg, wu, wd, x)) {
-    // hq_matmul_q_gated_act followed by hq_matmul_q_act, bit for bit: each half on the kernel that
-    // call would take.
-    auto *hact = static_cast<uint8_t *>(ws);
-    void *rest = static_cast<char *>(ws) + al256(4 * M * I);
-    if (skinny_gated_ok(M, I, H, dt, wg, wu, x)) {
-      float *h = static_cast<float *>(ws);
-      if (int rc = launch_skinny(x, wg, wu, h, M, I, H, act, dt, rest, s)) return rc;
-      // (The down projection's conversion of x takes h through its quantization itself.)
-      if (skinny_ok(M, H, I, dt, wd, h)) return launch_skinny_act(h, false, wd, out, M, H, I, dt, rest, s);
-      if (int rc = launch_quantize_act(h, F32, rest, M, I, s)) return rc;
-      return launch_gemv_q4kx_act(rest, wd, out, M, H, I, dt, s);
-    }
-    // Launch 1: gated gate/up on x, output quantized straight into ws (act layout of (M, I)).
-    if (int rc = launch_matmul_q_gated_act(x, wg, wu, hact, M, I, H, dt, act, nullptr, s)) return rc;
+  if (mlp_fused_ok(M, H, I, dt, wg, wu, wd, x) && !skinny_gated_ok(M, I, H, dt, wg, wu, x) &&
+      !skinny_ok(M, H, I, dt, wd, ws)) {
+    // Both halves on the int8 GEMV.  Launch 1: gated gate/up on x, output quantized straight into ws
+    // (act layout of (M, I)).
+    auto *h = static_cast<uint8_t *>(ws);
+    if (int rc = launch_matmul_q_gated_act(x, wg, wu, h, M, I, H, dt, act, nullptr, s)) return rc;
     // Launch 2: down projection on the prepared h.
-    if (skinny_ok(M, H, I, dt, wd, hact)) return launch_skinny_act(hact, true, wd, out, M, H, I, dt, rest, s);
-    return launch_gemv_q4kx_act(hact, wd, out, M, H, I, dt, s);
+    return launch_gemv_q4kx_act(h, wd, out, M, H, I, dt, s);
   }
   if (!skinny_ok(M, I, H, dt, wg, x) && !skinny_mid_ok(M, I, H, dt, wg, x)) {
     if (gemm_path(M, H) && gemm_path(M, I)) {

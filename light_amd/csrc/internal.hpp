@@ -50,8 +50,6 @@ int launch_gemm_ws_bf16(const uint16_t *xb, const uint16_t *wb, float *out, floa
                         int64_t K, hipStream_t s);
 size_t matmul_q_ws_bytes(int64_t M, int64_t N, int64_t K, int dt);
 size_t matmul_act_ws_bytes(int64_t M, int64_t N, int64_t K, int dt);
-// hq_matmul_q_act can do without that workspace (the int8 GEMV in place of skinny.hip).
-bool matmul_act_ws_optional(int64_t M, int64_t K, int dt);
 int launch_matmul_q(const float *x, const void *w, float *out, int64_t M, int64_t N, int64_t K, int dt, void *ws,
                     hipStream_t s);
 // The many-row GEMMs (M > 8, K % 64 == 0) on shared bf16 x: two weights on one conversion of x, and
@@ -107,7 +105,7 @@ int launch_gemv_q4kx_act(const void *act_in, const void *w, float *out, int64_t 
 // (tmp: M * N floats).
 bool q4kx_halves_ok(int64_t M, int64_t N, int64_t K, int dt, const void *w, const void *act);
 // The f16 MFMA product for a few rows of x (skinny.hip): Q4_K / Q5_K (w1 != NULL: gated) and
-// int4.  ws: skinny_ws_bytes (rows past 8192 only).
+// int4.  ws: skinny_ws_bytes (rows past 4096 only).
 constexpr int64_t kSkinnyMaxRows = 16;
 // (A row's x record stays below 1 MiB, the library workspace's first size.)
 constexpr int64_t kSkinnyMaxK = 29696;
@@ -117,8 +115,8 @@ bool skinny_int4_ok(int64_t M, int64_t N, int64_t K, int G, int x_dtype, const v
 size_t skinny_ws_bytes(int64_t M, int64_t K, bool int4);
 int launch_skinny(const float *x, const void *w0, const void *w1, float *out, int64_t M, int64_t N, int64_t K, int act,
                   int dt, void *ws, hipStream_t s);
-int launch_skinny_act(const void *x, bool prepared, const void *w, float *out, int64_t M, int64_t N, int64_t K, int dt,
-                      void *ws, hipStream_t s);
+// x as prepared activations: M <= 8, K <= 4096 (no workspace).
+int launch_skinny_act(const void *x, const void *w, float *out, int64_t M, int64_t N, int64_t K, int dt, hipStream_t s);
 // 17 to 64 rows (ws: skinny_mid_ws_bytes).
 bool skinny_mid_ok(int64_t M, int64_t N, int64_t K, int dt, const void *w, const void *x);
 size_t skinny_mid_ws_bytes(int64_t M, int64_t N, int64_t K);

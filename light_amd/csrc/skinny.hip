@@ -81,9 +81,8 @@ __device__ __forceinline__ f16x2 splat(float v) {
 
 }  // namespace
 
-// Sources of x besides the dtypes: prepared activations (act layout), and F32 taken through that
-// layout's quantization (the values hq_quantize_act + hq_matmul_q_act would use).
-constexpr int kXAct = -1, kXQuant = -2;
+// A source of x besides the dtypes: prepared activations (act layout).
+constexpr int kXAct = -1;
 
 struct SkinnyArgs {
   const void *x;           // (M, K) of x's dtype, or prepared activations
@@ -317,7 +316,7 @@ __device__ __forceinline__ void convert_row(const float (&v)[4], int m, int lane
 template <int XDT>
 __device__ __forceinline__ void load_x4(const SkinnyArgs &a, int m, int64_t k, float (&v)[4]) {
   const int64_t i = (int64_t)m * a.K + k;
-  if constexpr (XDT == F32 || XDT == kXQuant) {
+  if constexpr (XDT == F32) {
     const f32x4 f = *reinterpret_cast<const f32x4 *>(static_cast<const float *>(a.x) + i);
 #pragma unroll
     for (int j = 0; j < 4; j++) v[j] = f[j];
@@ -335,17 +334,6 @@ __device__ __forceinline__ void load_x4(const SkinnyArgs &a, int m, int64_t k, f
       const uint32_t h = (j & 1) ? u[j >> 1] >> 16 : u[j >> 1] & 0xffffu;
       v[j] = XDT == BF16 ? bf2f(h) : h2f(h);
     }
-  }
-}
-
-// kXQuant: the lane's four elements (eight lanes a block) as d q1 + e q2 of act_quant8.
-template <int XDT>
-__device__ __forceinline__ void through_act(float (&v)[4]) {
-  if constexpr (XDT == kXQuant) {
-    const ActQ q = act_quant8(v);
-#pragma unroll
-    for (int j = 0; j < 4; j++)
-      v[j] = __fmaf_rn(q.e, (float)(int8_t)(q.q2 >> (8 * j)), __fmul_rn(q.d, (float)(int8_t)(q.q1 >> (8 * j))));
   }
 }
 
@@ -629,10 +617,7 @@ __global__ __launch_bounds__(1024) void skinny_kernel(SkinnyArgs a) {
       if (wave / T::CW == ph) {
         uint8_t *rec = conv + (wave % T::CW) * (UPG * R::BYTES);
 #pragma unroll
-        for (int m = 0; m < XR; m++) {
-          through_act<XDT>(xv[m]);
-          convert_row<F, XM>(xv[m], m, lane, rec, R::ROWS);
-        }
+        for (int m = 0; m < XR; m++) convert_row<F, XM>(xv[m], m, lane, rec, R::ROWS);
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 #pragma unroll
         for (int q = 0; q < UPG; q++) load_frag<F, XM>(rec + q * R::BYTES, lane, xf[q]);
@@ -860,7 +845,6 @@ __global__ __launch_bounds__(256) void skinny_x_kernel(SkinnyArgs a, uint8_t *xf
   k = k < a.K ? k : a.K - 4;  // (int4, an odd unit count: the record past the end is allocated)
   float v[4];
   load_x4<XDT>(a, m, k, v);
-  through_act<XDT>(v);
   const int P = R::rows(a.M);
   convert_row<F, XM>(v, m, lane, xf + (int64_t)c * (UPC * R::bytes(P)), P);
 }
@@ -1057,8 +1041,7 @@ constexpr int64_t kSkinnyResMaxK = 4096;  // longer rows: x prepared in the work
 template <class F, bool GATED, int XDT, int ODT>
 int run_any(const SkinnyArgs &a, bool pair, void *ws, hipStream_t s) {
   const bool lng = a.K > kSkinnyResMaxK;
-  if constexpr (XDT >= 0)
-    if (a.M > 8) return lng ? run_long<F, GATED, kX16, XDT, ODT>(a, ws, s) : run_resident<F, GATED, kX16, XDT, ODT>(a, s);
+  if (a.M > 8) return lng ? run_long<F, GATED, kX16, XDT, ODT>(a, ws, s) : run_resident<F, GATED, kX16, XDT, ODT>(a, s);
   constexpr int kPair = XDT == BF16 || XDT == F16 ? kXDup : kXPair;  // (16-bit x needs no second part)
   if (pair) return lng ? run_long<F, GATED, kPair, XDT, ODT>(a, ws, s) : run_resident<F, GATED, kPair, XDT, ODT>(a, s);
   return lng ? run_long<F, GATED, kXDup, XDT, ODT>(a, ws, s) : run_resident<F, GATED, kXDup, XDT, ODT>(a, s);
@@ -1145,17 +1128,14 @@ int launch_skinny(const float *x, const void *w0, const void *w1, float *out, in
   return w1 ? run_any<SkQk<false>, true, F32, F32>(a, pair, ws, s) : run_any<SkQk<false>, false, F32, F32>(a, pair, ws, s);
 }
 
-// x as prepared activations, or F32 x taken through their quantization (the same results); M <= 8.
-int launch_skinny_act(const void *x, bool prepared, const void *w, float *out, int64_t M, int64_t N, int64_t K, int dt,
-                      void *ws, hipStream_t s) {
+int launch_skinny_act(const void *x, const void *w, float *out, int64_t M, int64_t N, int64_t K, int dt, hipStream_t s) {
   SkinnyArgs a = skinny_args(x, w, out, M, N, K, dt);
   a.xdt = kXAct;
-  const bool pair = skinny_pair(K);
   if (dt == Q5_K)
-    return prepared ? run_any<SkQk<true>, false, kXAct, F32>(a, pair, ws, s)
-                    : run_any<SkQk<true>, false, kXQuant, F32>(a, pair, ws, s);
-  return prepared ? run_any<SkQk<false>, false, kXAct, F32>(a, pair, ws, s)
-                  : run_any<SkQk<false>, false, kXQuant, F32>(a, pair, ws, s);
+    return skinny_pair(K) ? run_resident<SkQk<true>, false, kXPair, kXAct, F32>(a, s)
+                          : run_resident<SkQk<true>, false, kXDup, kXAct, F32>(a, s);
+  return skinny_pair(K) ? run_resident<SkQk<false>, false, kXPair, kXAct, F32>(a, s)
+                        : run_resident<SkQk<false>, false, kXDup, kXAct, F32>(a, s);
 }
 
 // ---- 17 <= M <= 64, Q4_K / Q5_K (skinny_mid_kernel) ----

@@ -90,27 +90,46 @@ def test_gated(dev, dt, M, N, K):
     assert ((h.double() - silu * b).abs() <= bound).all()
 
 
-@pytest.mark.parametrize("M,H,I", [(3, 4096, 5120), (5, 2048, 8192), (8, 4096, 3072), (6, 8192, 2048), (4, 2048, 8192)])
+@pytest.mark.parametrize("M,H,I", [(3, 4096, 5120), (5, 2048, 8192), (8, 4096, 3072), (6, 8192, 2048), (4, 8192, 2048),
+                                   (4, 5120, 6144)])
 def test_mlp_equals_its_halves(dev, M, H, I):
-    """Each half of the block on the kernel its own call takes, whichever those are."""
+    """A block with either half on the f16 tiles is its two calls, whichever kernels those take, whatever
+    the workspace."""
     print(f"[case] skinny mlp M={M} H={H} I={I}", flush=True)
     (wg, _), (wu, _), (wd, _) = (_weight(hipq.Q4_K, r, c, dev, seed=i) for i, (r, c) in enumerate(((I, H), (I, H), (H, I))))
     x = torch.randn(M, H, device=dev, generator=torch.Generator(device=dev).manual_seed(M)) * 0.01
-    want = hipq.matmul_q_act(hipq.matmul_q_gated_act(x, wg, wu, I, H, hipq.Q4_K), wd, M, H, I, hipq.Q4_K)
+    want = hipq.matmul_q(hipq.matmul_q_gated(x, wg, wu, I, H, hipq.Q4_K), wd, H, I, hipq.Q4_K)
     assert torch.equal(hipq.mlp_q(x, wg, wu, wd, H, I, hipq.Q4_K), want)
+    ws = torch.empty(hipq.mlp_q_ws_bytes(M, H, I, hipq.Q4_K), dtype=torch.uint8, device=dev)
+    assert torch.equal(hipq.mlp_q(x, wg, wu, wd, H, I, hipq.Q4_K, ws=ws), want)
 
 
-@pytest.mark.parametrize("M,N,K", [(3, 2567, 4096), (8, 1536, 14336)])
-def test_prepared_without_workspace(dev, M, N, K):
-    """hq_matmul_q_act with a caller's workspace too small for x's records takes the int8 GEMV."""
-    print(f"[case] skinny act M={M} N={N} K={K}", flush=True)
-    w, wd = _weight(hipq.Q4_K, N, K, dev, seed=K)
+@pytest.mark.parametrize("dt", [hipq.Q4_K, hipq.Q5_K])
+@pytest.mark.parametrize("M,N,K", [(3, 2567, 4096), (8, 1536, 14336), (5, 1700, 6144), (4, 1600, 16640)])
+def test_prepared_whatever_the_workspace(dev, dt, M, N, K):
+    """hq_matmul_q_act asks for no workspace at 3 to 8 rows, writes none that it is given, and gives the
+    same bits with none, any, and under capture on a stream whose library workspace cannot grow."""
+    print(f"[case] skinny act dt={hipq.NAMES[dt]} M={M} N={N} K={K}", flush=True)
+    w, wd = _weight(dt, N, K, dev, seed=K)
     x = torch.randn(M, K, device=dev, generator=torch.Generator(device=dev).manual_seed(M))
     act = hipq.quantize_act(x)
-    y = hipq.matmul_q_act(act, w, M, N, K, hipq.Q4_K)
-    small = hipq.matmul_q_act(act, w, M, N, K, hipq.Q4_K, ws=torch.empty(16, dtype=torch.uint8, device=dev))
-    want = x.double() @ wd.t()
-    assert _err(y, want, x, wd) <= 3e-4 and _err(small, want, x, wd) <= 1e-3
+    assert hipq.lib().hq_matmul_q_act_ws_bytes(M, N, K, dt) == 0
+    y = hipq.matmul_q_act(act, w, M, N, K, dt)
+    for n in (16, 1 << 20):
+        ws = torch.full((n,), 171, dtype=torch.uint8, device=dev)
+        assert torch.equal(hipq.matmul_q_act(act, w, M, N, K, dt, ws=ws), y)
+        assert (ws == 171).all(), "the caller's buffer was written"
+    out, g, s = torch.empty_like(y), torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s), torch.cuda.graph(g, stream=s):
+        hipq.matmul_q_act(act, w, M, N, K, dt, out=out)
+    for _ in range(3):
+        out.fill_(float("nan"))
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, y)
+    # (x by q8_1: 1e-3 from K = 4096 on where the GEMV reads one level.)
+    assert _err(y, x.double() @ wd.t(), x, wd) <= 1e-3
 
 
 @pytest.mark.parametrize("xdt,tol", [(torch.float32, 2e-5), (torch.bfloat16, 2.0 ** -8), (torch.float16, 2.0 ** -10)])

@@ -138,15 +138,15 @@ struct WsInt4 {
                                  float out_hi[16]) {
     const u32x4 q = *reinterpret_cast<const u32x4 *>(raw + (32 * h + r) * 16);
     const float s = reinterpret_cast<const float *>(raw + 1024)[r];
-    // s q - s z in one FMA, the quants as bytes (one mask per four, v_cvt_f32_ubyteN): the weight
-    // is rounded to bf16 next, so this is not the bit-exact dequant.
-    const float nz = -s * reinterpret_cast<const float *>(raw + 1024)[32 + r];
+    const float z = reinterpret_cast<const float *>(raw + 1024)[32 + r];
+    // The exact weight s (q - z), rounded once to f32 and once to bf16; the quants as bytes (one mask
+    // per four, v_cvt_f32_ubyteN).
 #pragma unroll
     for (int k = 0; k < 4; k++) {
       const uint32_t ev = q[k] & 0x0F0F0F0Fu, od = (q[k] >> 4) & 0x0F0F0F0Fu;
 #pragma unroll
       for (int j = 0; j < 8; j++) {
-        const float v = __fmaf_rn(s, (float)((((j & 1) ? od : ev) >> (8 * (j >> 1))) & 0xffu), nz);
+        const float v = s * ((float)((((j & 1) ? od : ev) >> (8 * (j >> 1))) & 0xffu) - z);
         if (k < 2)
           out_lo[8 * k + j] = v;
         else

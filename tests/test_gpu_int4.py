@@ -233,3 +233,25 @@ def test_matmul_int4_f16_split_k_streams_and_repeats(dev, M, N, K, G):
     torch.cuda.synchronize()
     for y in again + outs:
         assert torch.equal(y, first)
+
+
+@pytest.mark.parametrize("xdt", [hipq.F32, hipq.BF16, hipq.F16])
+@pytest.mark.parametrize("M,N,K", [(65, 130, 1024), (129, 1000, 448), (300, 257, 4096)])
+def test_prefill_weights_are_s_times_q_minus_z(dev, xdt, M, N, K):
+    """The many-row GEMM takes s (q - z) as it stands, for scales that are no f16 values too: codes that
+    equal their zero weigh exactly 0, and one other code per row is the whole of the result."""
+    print(f"[case] int4 exact zeros M={M} N={N} K={K} x={hipq.NAMES[xdt]}", flush=True)
+    rng = np.random.default_rng(M)
+    s = (rng.random((N, K // 64)) * 0.02 + 1e-3).astype(np.float32)
+    z = rng.integers(1, 16, size=(N, K // 64)).astype(np.float32)
+    codes = np.repeat(z.astype(np.uint32) * np.uint32(0x11111111), 8, axis=1)
+    x = torch.randn(M, K, device=dev, generator=torch.Generator(device=dev).manual_seed(M)).to(torch.bfloat16).to(TDT[xdt])
+    zero = hipq.int4_matmul(x, _t(codes, dev).view(torch.int32), _t(s, dev), _t(z, dev), 64)
+    assert torch.count_nonzero(zero) == 0
+    # Column c = row % K: its first nibble one below the zero, so w = -s there, rounded to bf16.
+    n = np.arange(N)
+    c = 8 * (n % (K // 8))
+    codes[n, c // 8] -= 1
+    y = hipq.int4_matmul(x, _t(codes, dev).view(torch.int32), _t(s, dev), _t(z, dev), 64)
+    want = -x[:, torch.from_numpy(c).to(dev)].float() * _t(s[n, c // 64], dev).to(torch.bfloat16).float()
+    assert torch.equal(y, want.to(TDT[xdt]))

@@ -395,15 +395,13 @@ __device__ __forceinline__ void unit_mma(const typename F::Raw &w, const XFrag<F
   }
 }
 
-// Output (m, n) over the columns [k0, k1) of w, from its f16 form y.  That form splits a weight into
-// sc * q and a minimum (int4: q and z), so an infinite x meets them as Inf - Inf.  A y that is not
-// finite is therefore worked out again as f32 arithmetic has it: x's non-finite elements times their
-// weights (the finite ones add nothing to those); without such an element y stands.  One compare per
-// output otherwise.
+// x's non-finite elements of row m in [k0, k1) times their weights of row n, if there are any.  An
+// infinite x meets the split weights (sc * q and a minimum; int4: q and z) as Inf - Inf, so an output
+// that is not finite is worked out again from these, as f32 arithmetic has it (the finite elements add
+// nothing to them): by one pass at the kernel's end, for the threads that saw such an output.
 template <class F>
-__device__ __forceinline__ float settle(const SkinnyArgs &a, const uint8_t *w, int m, int n, int k0, int k1, float y) {
-  if (__builtin_expect(__builtin_isfinite(y) || a.xdt < 0, 1)) return y;
-  float s = 0.f;
+__device__ __forceinline__ bool nonfinite_sum(const SkinnyArgs &a, const uint8_t *w, int m, int n, int k0, int k1, float &s) {
+  s = 0.f;
   bool any = false;
 #pragma unroll 1
   for (int k = k0; k < k1 && s == s; k += 8) {  // (NaN stays NaN)
@@ -440,7 +438,7 @@ __device__ __forceinline__ float settle(const SkinnyArgs &a, const uint8_t *w, i
     for (int j = 0; j < 8; j++)
       if (!__builtin_isfinite(v[j])) s += v[j] * d[j];
   }
-  return any ? s : y;
+  return any;
 }
 
 template <int ODT>
@@ -451,6 +449,18 @@ __device__ __forceinline__ void store_y(void *out, int64_t i, float y) {
     static_cast<uint16_t *>(out)[i] = f2bf_rne(y);
   else
     static_cast<uint16_t *>(out)[i] = f2h_rne(y);
+}
+
+// Output (m, n) again, where row m of x holds a non-finite element (gate and up both have it then).
+template <class F, bool GATED, int ODT>
+__device__ __forceinline__ void settle(const SkinnyArgs &a, int m, int n) {
+  float y, u;
+  if (m >= a.M || n >= a.N || !nonfinite_sum<F>(a, a.w0, m, n, 0, a.K, y)) return;
+  if constexpr (GATED) {
+    nonfinite_sum<F>(a, a.w1, m, n, 0, a.K, u);
+    y = gate_act(y, a.act) * u;
+  }
+  store_y<ODT>(a.out, (int64_t)m * a.N + n, y);
 }
 
 // A direct load of 16 bytes per lane from base + off (base uniform).
@@ -629,6 +639,7 @@ __global__ __launch_bounds__(1024) void skinny_kernel(SkinnyArgs a) {
 
   float *part = reinterpret_cast<float *>(smem + NS * T::STAGE);
   float gs[NO];
+  bool bad = false;  // an output of this thread is not finite
   // Outputs of (iteration, weight j): sums the KW parts of (tile, x row, weight row) in order; the
   // gate's sums wait in registers for the up weight's.
   auto reduce = [&](int it, int j, int buf) __attribute__((always_inline)) {
@@ -641,12 +652,11 @@ __global__ __launch_bounds__(1024) void skinny_kernel(SkinnyArgs a) {
       const int c = o & 15, m = (o >> 4) & (XROWS - 1), q = (o >> 4) / XROWS;
       float y = sum_parts<KW, XM>(pb + q * KW * 256, c, m);
       const int col = row0 + q * 16 + c;
-      if (m >= a.M || col >= a.N) continue;
-      if constexpr (XDT >= 0) y = settle<F>(a, GATED && j ? a.w1 : a.w0, m, col, 0, a.K, y);
       if (GATED && j == 0) {
         gs[k] = y;
-      } else {
+      } else if (m < a.M && col < a.N) {
         if constexpr (GATED) y = gate_act(gs[k], a.act) * y;
+        bad |= !__builtin_isfinite(y);
         store_y<ODT>(a.out, (int64_t)m * a.N + col, y);
       }
     }
@@ -677,6 +687,14 @@ __global__ __launch_bounds__(1024) void skinny_kernel(SkinnyArgs a) {
   __syncthreads();
   reduce(niter - 1, NW - 1, NW == 2 ? 1 : (niter - 1) & 1);
   wait_vm<0>();  // the last (repeated) stages have landed before the LDS is given up
+  if constexpr (XDT >= 0)
+    if (bad) {
+#pragma unroll 1
+      for (int it = 0; it < niter; it++)
+#pragma unroll 1
+        for (int o = t; o < TG * 16 * XROWS; o += 1024)
+          settle<F, GATED, ODT>(a, (o >> 4) & (XROWS - 1), row0_of(it) + (o >> 4) / XROWS * 16 + (o & 15));
+    }
 }
 
 // Longer rows: RT tiles per workgroup, x from skinny_x_kernel's records.  Items are (K chunk of up
@@ -811,6 +829,7 @@ __global__ __launch_bounds__(1024) void skinny_long_kernel(SkinnyArgs a) {
   }
   float *part = reinterpret_cast<float *>(smem);
   float gs = 0.f;
+  bool bad = false;
 #pragma unroll
   for (int k = 0; k < NT; k++) {
     __syncthreads();  // (first: every wave is done with the stages; then: the part before was summed)
@@ -818,16 +837,19 @@ __global__ __launch_bounds__(1024) void skinny_long_kernel(SkinnyArgs a) {
     __syncthreads();
     if (t < 16 * XROWS) {
       const int c = t & 15, m = t >> 4, col = row0_of(k / NW) + c;
-      if (m < a.M && col < a.N) {
-        float y = settle<F>(a, k % NW ? a.w1 : a.w0, m, col, 0, a.K, sum_parts<CW, XM>(part, c, m));
-        if (GATED && k % NW == 0) {
-          gs = y;
-        } else {
-          if constexpr (GATED) y = gate_act(gs, a.act) * y;
-          store_y<ODT>(a.out, (int64_t)m * a.N + col, y);
-        }
+      float y = sum_parts<CW, XM>(part, c, m);
+      if (GATED && k % NW == 0) {
+        gs = y;
+      } else if (m < a.M && col < a.N) {
+        if constexpr (GATED) y = gate_act(gs, a.act) * y;
+        bad |= !__builtin_isfinite(y);
+        store_y<ODT>(a.out, (int64_t)m * a.N + col, y);
       }
     }
+  }
+  if (bad) {
+#pragma unroll 1
+    for (int i = 0; i < RT; i++) settle<F, GATED, ODT>(a, t >> 4, row0_of(i) + (t & 15));
   }
 }
 
@@ -948,14 +970,26 @@ __global__ __launch_bounds__(512) void skinny_mid_kernel(SkinnyArgs a) {
   wait_vm<0>();
   float *out = static_cast<float *>(a.out) + (int64_t)blockIdx.y * a.M * a.N;
   const int col = row0 + r;
+  bool bad = false;
   if (col < a.N) {
 #pragma unroll
     for (int m = 0; m < MT; m++)
 #pragma unroll
       for (int j = 0; j < 4; j++) {
         const int row = m * 16 + 4 * g + j;
-        if (row < a.M) out[(int64_t)row * a.N + col] = settle<F>(a, a.w0, row, col, u0 * 256, u1 * 256, acc[m][j]);
+        if (row < a.M) {
+          out[(int64_t)row * a.N + col] = acc[m][j];
+          bad |= !__builtin_isfinite(acc[m][j]);
+        }
       }
+    if (bad) {
+#pragma unroll 1
+      for (int i = 0; i < 4 * MT; i++) {
+        const int row = (i >> 2) * 16 + 4 * g + (i & 3);
+        float y;
+        if (row < a.M && nonfinite_sum<F>(a, a.w0, row, col, u0 * 256, u1 * 256, y)) out[(int64_t)row * a.N + col] = y;
+      }
+    }
   }
 }
 

@@ -612,28 +612,48 @@ __global__ __launch_bounds__(1024) void skinny_kernel(SkinnyArgs a) {
 #pragma unroll
   for (int i = 0; i < NS - 1; i++) issue(i / NW, i % NW, i);
 
-  // The wave's group of x (units kw UPG ..).  XR rows are converted without a branch between them,
-  // so that their chains interleave (rows past M repeat row M - 1).
+  // The wave's group of x (units kw UPG ..).  Rows are converted without a branch between them, so that
+  // their chains interleave (rows past M repeat row M - 1).
   XFrag<F> xf[UPG];
   {
     uint8_t *conv = smem + 2 * T::STAGE;
-    float xv[XR][4];
     int64_t k = (int64_t)kw * 256 + lane * 4;
     k = k < a.K ? k : a.K - 4;
+    auto load_frags = [&](const uint8_t *rec) __attribute__((always_inline)) {
 #pragma unroll
-    for (int m = 0; m < XR; m++) load_x4<XDT>(a, m < a.M ? m : a.M - 1, k, xv[m]);
+      for (int q = 0; q < UPG; q++) load_frag<F, XM>(rec + q * R::BYTES, lane, xf[q]);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    };
+    if constexpr (TG > 1) {
+      // The TG waves of a group convert XR / TG of its rows each (M = 16, 4345 x 256: 12.6 us with every
+      // wave converting all rows of its group, 5.6 so; M = 9, 12357 x 512, Q5_K: 12.7, 6.1).
+      constexpr int RW = (XR + TG - 1) / TG;
+      uint8_t *rec = conv + kw * (UPG * R::BYTES);
+      float xv[RW][4];
 #pragma unroll
-    for (int ph = 0; ph < 16 / T::CW; ph++) {
-      if (wave / T::CW == ph) {
-        uint8_t *rec = conv + (wave % T::CW) * (UPG * R::BYTES);
+      for (int i = 0; i < RW; i++) load_x4<XDT>(a, tg + i * TG < a.M ? tg + i * TG : a.M - 1, k, xv[i]);
+      if (XR >= TG || tg < XR) {
 #pragma unroll
-        for (int m = 0; m < XR; m++) convert_row<F, XM>(xv[m], m, lane, rec, R::ROWS);
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-#pragma unroll
-        for (int q = 0; q < UPG; q++) load_frag<F, XM>(rec + q * R::BYTES, lane, xf[q]);
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        for (int i = 0; i < RW; i++) convert_row<F, XM>(xv[i], tg + i * TG, lane, rec, R::ROWS);
       }
-      __syncthreads();  // the next waves' records, then the stage and the parts, take the place
+      __syncthreads();
+      load_frags(rec);
+      __syncthreads();  // the stage and the parts take the place
+    } else {
+      float xv[XR][4];
+#pragma unroll
+      for (int m = 0; m < XR; m++) load_x4<XDT>(a, m < a.M ? m : a.M - 1, k, xv[m]);
+#pragma unroll
+      for (int ph = 0; ph < 16 / T::CW; ph++) {
+        if (wave / T::CW == ph) {
+          uint8_t *rec = conv + (wave % T::CW) * (UPG * R::BYTES);
+#pragma unroll
+          for (int m = 0; m < XR; m++) convert_row<F, XM>(xv[m], m, lane, rec, R::ROWS);
+          asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+          load_frags(rec);
+        }
+        __syncthreads();  // the next waves' records, then the stage and the parts, take the place
+      }
     }
   }
 

@@ -29,6 +29,15 @@ def _weight(dt, N, K, dev, seed):
     return w, hipq.dequant(w, N * K, dt).view(N, K).double()
 
 
+def _big_weight(dt, N, K, dev):
+    """Random quants under one small scale, made on the GPU."""
+    per, size = hipq.BLOCK[dt]
+    g = torch.Generator(device=dev).manual_seed(N + K)
+    w = torch.randint(0, 256, (N * K // per, size), dtype=torch.uint8, device=dev, generator=g)
+    w[:, 0:4] = torch.tensor([1e-4, 7e-4], dtype=torch.float16, device=dev).view(torch.uint8)
+    return w
+
+
 def _err(y, want, x, wd):
     scale = torch.outer(x.double().norm(dim=1), wd.norm(dim=1))
     return ((y.double() - want).abs() / scale).max().item()
@@ -130,6 +139,38 @@ def test_prepared_whatever_the_workspace(dev, dt, M, N, K):
         assert torch.equal(out, y)
     # (x by q8_1: 1e-3 from K = 4096 on where the GEMV reads one level.)
     assert _err(y, x.double() @ wd.t(), x, wd) <= 1e-3
+
+
+@pytest.mark.parametrize("xdt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("M", [3, 4, 7, 9, 15, 16])
+@pytest.mark.parametrize("K", [128, 256, 384, 512, 1024, 1152, 2048])
+def test_int4_short_rows(dev, xdt, M, K):
+    """Rows of one to eight groups of 256, whose x the waves of a group convert together (M = 9 to 16 from
+    the rule's 30M and 40M weights)."""
+    N, G = (45000000 if M > 8 else 12600000) // K + 5, 128
+    print(f"[case] skinny int4 short x={xdt} M={M} N={N} K={K}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(K)
+    codes = torch.randint(-2 ** 31, 2 ** 31, (N, K // 8), dtype=torch.int64, device=dev, generator=g).to(torch.int32)
+    s, z = torch.rand(N, K // G, device=dev, generator=g) * 0.01 + 1e-3, torch.randint(0, 16, (N, K // G), device=dev, generator=g).float()
+    x = torch.randn(M, K, device=dev, generator=g).to(xdt)
+    wd = hipq.int4_dequant(codes, s, z, G).double()
+    tol = 2.0 ** -8 if xdt == torch.bfloat16 else 2.5e-4 if M > 8 else 2e-5
+    assert _err(hipq.int4_matmul(x, codes, s, z, G), x.double() @ wd.t(), x, wd) <= tol
+
+
+@pytest.mark.parametrize("dt", [hipq.Q4_K, hipq.Q5_K])
+@pytest.mark.parametrize("M", [3, 4, 7, 8, 9, 13, 16])
+@pytest.mark.parametrize("K", [256, 512, 768, 1024, 1280, 2048])
+def test_short_rows(dev, dt, M, K):
+    """The same for the K formats, with x of every scale."""
+    N = 10000000 // K + 21
+    print(f"[case] skinny short dt={hipq.NAMES[dt]} M={M} N={N} K={K}", flush=True)
+    w = _big_weight(dt, N, K, dev)
+    wd = hipq.dequant(w, N * K, dt).view(N, K).double()
+    x = _x(M, K, dev, seed=M)
+    y = hipq.matmul_q(x, w, N, K, dt)
+    assert _err(y, x.double() @ wd.t(), x, wd) <= (2e-5 if M <= 8 else 2.5e-4)
+    assert torch.equal(y, hipq.matmul_q(x, w, N, K, dt)), "not deterministic"
 
 
 @pytest.mark.parametrize("xdt,tol", [(torch.float32, 2e-5), (torch.bfloat16, 2.0 ** -8), (torch.float16, 2.0 ** -10)])

@@ -179,10 +179,11 @@ int hq_matmul_q_gated_act(const float *x, const void *wg, const void *wu, void *
 /* The gated MLP block of a decoder layer:
  *   out (M, H) F32 = (act(x @ dequant(wg)^T) * (x @ dequant(wu)^T)) @ dequant(wd)^T
  * with x (M, H) F32, wg and wu (I, H), wd (H, I), all of w_dtype; act as above.
- * For Q4_K / Q5_K with M <= 8 where both halves take the int8 GEMV (M <= 2, and small weights) this
- * is two launches, hq_matmul_q_gated_act (the gated gate/up GEMV, which writes its output already
- * quantized for the next matmul into ws) and hq_matmul_q_act (the down GEMV on it), bit for bit.
- * Other cases run hq_matmul_q_gated into ws and then hq_matmul_q, bit for bit.
+ * For Q4_K / Q5_K with M <= 8 whose gate/up takes the int8 GEMV (M <= 2, small weights, other rows at
+ * M <= 4 than 2048 < H <= 4096) that GEMV writes h already quantized for the next matmul into ws, as
+ * hq_matmul_q_gated_act does, and the down projection runs on it: hq_matmul_q_act, bit for bit, or at
+ * M >= 3 past I = 4096 its f16 MFMA form.  Other cases run hq_matmul_q_gated into ws and then hq_matmul_q,
+ * bit for bit.
  * Light: models/llama.go:1306-1333 (GatedLinear or MatMulQ/SiLU/Mul, then DownProj).
  * No counterpart op in Light. */
 size_t hq_mlp_q_ws_bytes(int64_t M, int64_t H, int64_t I, int w_dtype);

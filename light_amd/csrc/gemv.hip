@@ -1253,7 +1253,7 @@ int launch_matmul_act(const void *act, const void *w, float *out, int64_t M, int
     return launch_gemv_q4kx_act_halves(act, w, out, static_cast<float *>(ws), M, N, K, dt, s);
   // (Longer rows would need a workspace for x's records, which this call has none for: the GEMV.)
   if (M <= kGemvMaxRows && skinny_ws_bytes(M, K, false) == 0 && skinny_ok(M, N, K, dt, w, act))
-    return launch_skinny_act(act, w, out, M, N, K, dt, s);
+    return launch_skinny_act(act, w, out, M, N, K, dt, nullptr, s);
   return launch_gemv_act(act, w, out, M, N, K, dt, s);
 }
 

@@ -2718,13 +2718,14 @@ int launch_matmul_q_gated_act(const float *x, const void *wg, const void *wu, ui
 
 int launch_mlp_q(const float *x, const void *wg, const void *wu, const void *wd, float *out, int64_t M, int64_t H,
                  int64_t I, int dt, int act, void *ws, hipStream_t s) {
-  if (mlp_fused_ok(M, H, I, dt, wg, wu, wd, x) && !skinny_gated_ok(M, I, H, dt, wg, wu, x) &&
-      !skinny_ok(M, H, I, dt, wd, ws)) {
-    // Both halves on the int8 GEMV.  Launch 1: gated gate/up on x, output quantized straight into ws
-    // (act layout of (M, I)).
+  if (mlp_fused_ok(M, H, I, dt, wg, wu, wd, x) && !skinny_gated_ok(M, I, H, dt, wg, wu, x)) {
+    // Launch 1: gated gate/up GEMV on x, output quantized straight into ws (act layout of (M, I)).
     auto *h = static_cast<uint8_t *>(ws);
     if (int rc = launch_matmul_q_gated_act(x, wg, wu, h, M, I, H, dt, act, nullptr, s)) return rc;
-    // Launch 2: down projection on the prepared h.
+    // Launch 2: down projection on the prepared h.  (Long rows: x's records behind it, where I >= 4352 and
+    // so act_bytes(M, I) < 4 M I.)
+    if (skinny_ok(M, H, I, dt, wd, h))
+      return launch_skinny_act(h, wd, out, M, H, I, dt, static_cast<char *>(ws) + al256(4 * M * I), s);
     return launch_gemv_q4kx_act(h, wd, out, M, H, I, dt, s);
   }
   if (!skinny_ok(M, I, H, dt, wg, x) && !skinny_mid_ok(M, I, H, dt, wg, x)) {

@@ -115,8 +115,9 @@ bool skinny_int4_ok(int64_t M, int64_t N, int64_t K, int G, int x_dtype, const v
 size_t skinny_ws_bytes(int64_t M, int64_t K, bool int4);
 int launch_skinny(const float *x, const void *w0, const void *w1, float *out, int64_t M, int64_t N, int64_t K, int act,
                   int dt, void *ws, hipStream_t s);
-// x as prepared activations: M <= 8, K <= 4096 (no workspace).
-int launch_skinny_act(const void *x, const void *w, float *out, int64_t M, int64_t N, int64_t K, int dt, hipStream_t s);
+// x as prepared activations, M <= 8.
+int launch_skinny_act(const void *x, const void *w, float *out, int64_t M, int64_t N, int64_t K, int dt, void *ws,
+                      hipStream_t s);
 // 17 to 64 rows (ws: skinny_mid_ws_bytes).
 bool skinny_mid_ok(int64_t M, int64_t N, int64_t K, int dt, const void *w, const void *x);
 size_t skinny_mid_ws_bytes(int64_t M, int64_t N, int64_t K);

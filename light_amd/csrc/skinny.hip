@@ -867,7 +867,7 @@ __global__ __launch_bounds__(1024) void skinny_long_kernel(SkinnyArgs a) {
       }
     }
   }
-  if (bad) {
+  if (bad && a.xdt >= 0) {
 #pragma unroll 1
     for (int i = 0; i < RT; i++) settle<F, GATED, ODT>(a, t >> 4, row0_of(i) + (t & 15));
   }
@@ -1095,7 +1095,8 @@ constexpr int64_t kSkinnyResMaxK = 4096;  // longer rows: x prepared in the work
 template <class F, bool GATED, int XDT, int ODT>
 int run_any(const SkinnyArgs &a, bool pair, void *ws, hipStream_t s) {
   const bool lng = a.K > kSkinnyResMaxK;
-  if (a.M > 8) return lng ? run_long<F, GATED, kX16, XDT, ODT>(a, ws, s) : run_resident<F, GATED, kX16, XDT, ODT>(a, s);
+  if constexpr (XDT >= 0)
+    if (a.M > 8) return lng ? run_long<F, GATED, kX16, XDT, ODT>(a, ws, s) : run_resident<F, GATED, kX16, XDT, ODT>(a, s);
   constexpr int kPair = XDT == BF16 || XDT == F16 ? kXDup : kXPair;  // (16-bit x needs no second part)
   if (pair) return lng ? run_long<F, GATED, kPair, XDT, ODT>(a, ws, s) : run_resident<F, GATED, kPair, XDT, ODT>(a, s);
   return lng ? run_long<F, GATED, kXDup, XDT, ODT>(a, ws, s) : run_resident<F, GATED, kXDup, XDT, ODT>(a, s);
@@ -1182,14 +1183,12 @@ int launch_skinny(const float *x, const void *w0, const void *w1, float *out, in
   return w1 ? run_any<SkQk<false>, true, F32, F32>(a, pair, ws, s) : run_any<SkQk<false>, false, F32, F32>(a, pair, ws, s);
 }
 
-int launch_skinny_act(const void *x, const void *w, float *out, int64_t M, int64_t N, int64_t K, int dt, hipStream_t s) {
+int launch_skinny_act(const void *x, const void *w, float *out, int64_t M, int64_t N, int64_t K, int dt, void *ws,
+                      hipStream_t s) {
   SkinnyArgs a = skinny_args(x, w, out, M, N, K, dt);
   a.xdt = kXAct;
-  if (dt == Q5_K)
-    return skinny_pair(K) ? run_resident<SkQk<true>, false, kXPair, kXAct, F32>(a, s)
-                          : run_resident<SkQk<true>, false, kXDup, kXAct, F32>(a, s);
-  return skinny_pair(K) ? run_resident<SkQk<false>, false, kXPair, kXAct, F32>(a, s)
-                        : run_resident<SkQk<false>, false, kXDup, kXAct, F32>(a, s);
+  const bool pair = skinny_pair(K);
+  return dt == Q5_K ? run_any<SkQk<true>, false, kXAct, F32>(a, pair, ws, s) : run_any<SkQk<false>, false, kXAct, F32>(a, pair, ws, s);
 }
 
 // ---- 17 <= M <= 64, Q4_K / Q5_K (skinny_mid_kernel) ----

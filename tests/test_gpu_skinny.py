@@ -102,15 +102,24 @@ def test_gated(dev, dt, M, N, K):
 @pytest.mark.parametrize("M,H,I", [(3, 4096, 5120), (5, 2048, 8192), (8, 4096, 3072), (6, 8192, 2048), (4, 8192, 2048),
                                    (4, 5120, 6144)])
 def test_mlp_equals_its_halves(dev, M, H, I):
-    """A block with either half on the f16 tiles is its two calls, whichever kernels those take, whatever
-    the workspace."""
+    """A block is its two calls, whichever kernels those take, whatever the workspace: on F32 h where the
+    gated call takes the f16 tiles, on quantized h where it takes the GEMV.  (Past I = 4096 the down half
+    takes the tiles on that h, which is its F32 form to 2^-15.)"""
     print(f"[case] skinny mlp M={M} H={H} I={I}", flush=True)
     (wg, _), (wu, _), (wd, _) = (_weight(hipq.Q4_K, r, c, dev, seed=i) for i, (r, c) in enumerate(((I, H), (I, H), (H, I))))
     x = torch.randn(M, H, device=dev, generator=torch.Generator(device=dev).manual_seed(M)) * 0.01
-    want = hipq.matmul_q(hipq.matmul_q_gated(x, wg, wu, I, H, hipq.Q4_K), wd, H, I, hipq.Q4_K)
-    assert torch.equal(hipq.mlp_q(x, wg, wu, wd, H, I, hipq.Q4_K), want)
+    h = hipq.matmul_q_gated(x, wg, wu, I, H, hipq.Q4_K)
+    got = hipq.mlp_q(x, wg, wu, wd, H, I, hipq.Q4_K)
+    if M > 4 or H <= 4096:
+        assert torch.equal(got, hipq.matmul_q(h, wd, H, I, hipq.Q4_K))
+    elif I <= 4096:
+        act = hipq.matmul_q_gated_act(x, wg, wu, I, H, hipq.Q4_K)
+        assert torch.equal(got, hipq.matmul_q_act(act, wd, M, H, I, hipq.Q4_K))
+    else:
+        wdd = hipq.dequant(wd, H * I, hipq.Q4_K).view(H, I).double()
+        assert _err(got, h.double() @ wdd.t(), h, wdd) <= 2.5e-4
     ws = torch.empty(hipq.mlp_q_ws_bytes(M, H, I, hipq.Q4_K), dtype=torch.uint8, device=dev)
-    assert torch.equal(hipq.mlp_q(x, wg, wu, wd, H, I, hipq.Q4_K, ws=ws), want)
+    assert torch.equal(hipq.mlp_q(x, wg, wu, wd, H, I, hipq.Q4_K, ws=ws), got)
 
 
 @pytest.mark.parametrize("dt", [hipq.Q4_K, hipq.Q5_K])

@@ -1062,6 +1062,23 @@ int run_resident(const SkinnyArgs &a, hipStream_t s) {
   }
 }
 
+// Tiles per workgroup of skinny_long_kernel: 1, 2 or 4, or where that leaves CUs idle (rounds of
+// workgroups, one per CU, times their tiles and one for a round's start) 3, 5 or 6.  With four, 16896 x
+// 8192 (1056 tiles, M = 4) was 264 workgroups, two rounds: 35.3 us, 26.7 with five; 8704 x 8192 half the
+// CUs: 19.2, 17.0 with three.  Gains of less than an eighth are none (45056 x 5632: 41.2 us with four, 43.1
+// with six).  (Gated: at most two of each weight, four spill.  Q5_K's six spill eight registers and are
+// still the faster ones: 21504 x 7680 41.1 us with four, 34.2.)
+int long_rt(int64_t tiles, bool gated) {
+  const int64_t cus = device_cus();
+  auto cost = [&](int c) { return cdiv(cdiv(tiles, c), cus) * (c + 1); };
+  int rt = tiles <= cus ? 1 : tiles <= 2 * cus ? 2 : 4;
+  if (gated) return std::min(rt, 2);
+  if (rt == 4)
+    for (int c : {3, 5, 6})
+      if (8 * cost(c) <= 7 * cost(4) && cost(c) < cost(rt)) rt = c;
+  return rt;
+}
+
 template <class F, int RT, bool GATED, int XM, int ODT>
 int run_skinny_long(const SkinnyArgs &a, hipStream_t s) {
   constexpr int lds = SkinnyLongLds<F>::BYTES;
@@ -1083,11 +1100,14 @@ int run_long(SkinnyArgs a, void *ws, hipStream_t s) {
   a.nch = (int)cdiv(nkg, T::CG);
   a.cg = (int)cdiv(nkg, a.nch);
   a.pr = a.cg * (T::GB / 16);
-  const int per = (int)cdiv(a.tiles, device_cus());
-  if (per <= 1) return run_skinny_long<F, 1, GATED, XM, ODT>(a, s);
-  if constexpr (!GATED)  // (four tiles of two weights spill)
-    if (per > 2) return run_skinny_long<F, 4, GATED, XM, ODT>(a, s);
-  return run_skinny_long<F, 2, GATED, XM, ODT>(a, s);
+  const int rt = long_rt(a.tiles, GATED);
+  if constexpr (!GATED) {
+    if (rt == 3) return run_skinny_long<F, 3, GATED, XM, ODT>(a, s);
+    if (rt == 4) return run_skinny_long<F, 4, GATED, XM, ODT>(a, s);
+    if (rt == 5) return run_skinny_long<F, 5, GATED, XM, ODT>(a, s);
+    if (rt == 6) return run_skinny_long<F, 6, GATED, XM, ODT>(a, s);
+  }
+  return rt == 1 ? run_skinny_long<F, 1, GATED, XM, ODT>(a, s) : run_skinny_long<F, 2, GATED, XM, ODT>(a, s);
 }
 
 constexpr int64_t kSkinnyResMaxK = 4096;  // longer rows: x prepared in the workspace

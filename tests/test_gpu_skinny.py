@@ -182,6 +182,37 @@ def test_short_rows(dev, dt, M, K):
     assert torch.equal(y, hipq.matmul_q(x, w, N, K, dt)), "not deterministic"
 
 
+# Tiles of the long kernel: from one up to six per workgroup, ragged last workgroups and a second round.
+LONG_N = [(3000, 4608), (5003, 4352), (10003, 4352), (14003, 4352), (18003, 4352), (22003, 4352), (30003, 4352)]
+
+
+@pytest.mark.parametrize("dt", [hipq.Q4_K, hipq.Q5_K])
+@pytest.mark.parametrize("M", [3, 8, 16])
+@pytest.mark.parametrize("N,K", LONG_N)
+def test_long_row_tiles(dev, dt, M, N, K):
+    print(f"[case] skinny long dt={hipq.NAMES[dt]} M={M} N={N} K={K}", flush=True)
+    w = _big_weight(dt, N, K, dev)
+    wd = hipq.dequant(w, N * K, dt).view(N, K).double()
+    x = _x(M, K, dev, seed=M)
+    y = hipq.matmul_q(x, w, N, K, dt)
+    assert _err(y, x.double() @ wd.t(), x, wd) <= 2.5e-4
+    assert torch.equal(y, hipq.matmul_q(x, w, N, K, dt)), "not deterministic"
+
+
+@pytest.mark.parametrize("xdt,tol", [(torch.float32, 2.5e-4), (torch.bfloat16, 2.0 ** -8), (torch.float16, 2.0 ** -10)])
+@pytest.mark.parametrize("M", [4, 13])
+@pytest.mark.parametrize("N,K", LONG_N)
+def test_int4_long_row_tiles(dev, xdt, tol, M, N, K):
+    print(f"[case] skinny int4 long x={xdt} M={M} N={N} K={K}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(N)
+    codes = torch.randint(-2 ** 31, 2 ** 31, (N, K // 8), dtype=torch.int64, device=dev, generator=g).to(torch.int32)
+    s, z = torch.rand(N, K // 128, device=dev, generator=g) * 0.01 + 1e-3, torch.rand(N, K // 128, device=dev, generator=g) * 15
+    x = torch.randn(M, K, device=dev, generator=g).to(xdt)
+    wd = hipq.int4_dequant(codes, s, z, 128).double()
+    # (M > 8 below the rule's size takes the bf16 GEMM: both operands rounded, 2^-8.)
+    assert _err(hipq.int4_matmul(x, codes, s, z, 128), x.double() @ wd.t(), x, wd) <= (tol if M <= 8 else 2.0 ** -8 + tol)
+
+
 @pytest.mark.parametrize("xdt,tol", [(torch.float32, 2e-5), (torch.bfloat16, 2.0 ** -8), (torch.float16, 2.0 ** -10)])
 @pytest.mark.parametrize("M", [3, 8, 16])
 @pytest.mark.parametrize("N,K,G", [(3208, 4096, 128), (3600, 3584, 256), (5000, 2688, 128), (4100, 4224, 128),

@@ -2722,9 +2722,12 @@ int launch_mlp_q(const float *x, const void *wg, const void *wu, const void *wd,
     // Launch 1: gated gate/up GEMV on x, output quantized straight into ws (act layout of (M, I)).
     auto *h = static_cast<uint8_t *>(ws);
     if (int rc = launch_matmul_q_gated_act(x, wg, wu, h, M, I, H, dt, act, nullptr, s)) return rc;
-    // Launch 2: down projection on the prepared h.  (Long rows: x's records behind it, where I >= 4352 and
-    // so act_bytes(M, I) < 4 M I.)
-    if (skinny_ok(M, H, I, dt, wd, h))
+    // Launch 2: down projection on the prepared h.  The f16 tiles (long rows: x's records behind h, where
+    // I >= 4352 and so act_bytes(M, I) < 4 M I), but for narrow blocks that one pass of the GEMV serves, whose
+    // 128 tiles leave half the CUs idle (M = 4, H x I = 2048 x 8192: 18.8 us, 23.7 with the tiles; 1536 x
+    // 16384 34.4, 37.0; past I = 16384 the GEMV slows: 2048 x 18944 46.4, 41.1).
+    const bool narrow = M <= 4 && H <= 2048 && I <= 16384;
+    if (!narrow && skinny_ok(M, H, I, dt, wd, h))
       return launch_skinny_act(h, wd, out, M, H, I, dt, static_cast<char *>(ws) + al256(4 * M * I), s);
     return launch_gemv_q4kx_act(h, wd, out, M, H, I, dt, s);
   }

@@ -227,3 +227,14 @@ def test_int4(dev, xdt, tol, M, N, K, G):
     wd = hipq.int4_dequant(codes, s, z, G).double()
     # (M > 8 below the rule's size takes the bf16 GEMM: both operands rounded, 2^-8.)
     assert _err(y, x.double() @ wd.t(), x, wd) <= (tol if M <= 8 else max(tol, 2.0 ** -8 + tol))
+
+
+@pytest.mark.parametrize("dt", [hipq.Q4_K, hipq.Q5_K])
+@pytest.mark.parametrize("M,H,I,gemv", [(3, 2048, 8192, True), (4, 1536, 16384, True), (4, 2048, 16640, False),
+                                        (4, 2304, 8192, False), (5, 2048, 8192, False)])
+def test_narrow_mlp_of_four_rows_takes_the_gemv(dev, dt, M, H, I, gemv):
+    print(f"[case] skinny route mlp dt={hipq.NAMES[dt]} M={M} H={H} I={I}", flush=True)
+    wg, wu, wd = (_big_weight(dt, r, c, dev) for r, c in ((I, H), (I, H), (H, I)))
+    x = torch.randn(M, H, device=dev, generator=torch.Generator(device=dev).manual_seed(M)) * 0.01
+    want = hipq.matmul_q_act(hipq.matmul_q_gated_act(x, wg, wu, I, H, dt), wd, M, H, I, dt)
+    assert torch.equal(hipq.mlp_q(x, wg, wu, wd, H, I, dt), want) == gemv

@@ -1079,6 +1079,12 @@ int long_rt(int64_t tiles, bool gated) {
   return rt;
 }
 
+// At most six tiles a CU, or the workgroups' rounds seven eighths full.
+bool long_few_or_full(int64_t tiles) {
+  const int64_t cus = device_cus(), rt = long_rt(tiles, false);
+  return tiles <= 6 * cus || 8 * tiles >= 7 * cdiv(cdiv(tiles, rt), cus) * cus * rt;
+}
+
 template <class F, int RT, bool GATED, int XM, int ODT>
 int run_skinny_long(const SkinnyArgs &a, hipStream_t s) {
   constexpr int lds = SkinnyLongLds<F>::BYTES;
@@ -1133,13 +1139,19 @@ int run_any(const SkinnyArgs &a, bool pair, void *ws, hipStream_t s) {
 //    need 96 tiles (1536 x 14336, M = 3: 15.2 / 14.4; 1024 x 16384: 11.4 / 16.2).
 //  * Gated at M <= 4: rows of (2048, 4096] only (the MLP of 2048 x 8192 at M = 3: 21.9 / 25.1 with
 //    both halves here; 4096 x 14336: 51.8 / 38.1).
+//    At M <= 4, one pass of the GEMV, past six tiles a CU only where the rounds of workgroups are nearly full
+//    (28672 x 8192 39.6 / 36.7; 25600 x 16384 54.0 / 58.1; 50426 x 4864 42.7 / 50.4), or Q4_K past 16384,
+//    where its GEMV slows (24576 x 18944: 146.5 / 70.2).
 //  * M > 8: always, against the GEMM's conversion, product and split-K launches (14336 x 4096,
 //    M = 12: 30.6 / 20.1; 1024 x 4096: 16.1 / 13.8).
 bool skinny_ok(int64_t M, int64_t N, int64_t K, int dt, const void *w, const void *x) {
   if ((dt != Q4_K && dt != Q5_K) || M < 3 || M > kSkinnyMaxRows || K <= 0 || K % 256 || K > kSkinnyMaxK || N < 1 ||
       (N + 64) * (K / 256) * block_info(dt).bytes > UINT32_MAX || ((uintptr_t)w & 15) || ((uintptr_t)x & 15))
     return false;
-  return M > 8 || (N * K >= 10000000 && (K <= kSkinnyResMaxK || N >= 1536));
+  if (M > 8) return true;
+  if (N * K < 10000000) return false;
+  if (K <= kSkinnyResMaxK) return true;
+  return N >= 1536 && (M > 4 || (dt == Q4_K && K > 16384) || long_few_or_full(cdiv(N, 16)));
 }
 
 bool skinny_gated_ok(int64_t M, int64_t N, int64_t K, int dt, const void *wg, const void *wu, const void *x) {
@@ -1147,21 +1159,34 @@ bool skinny_gated_ok(int64_t M, int64_t N, int64_t K, int dt, const void *wg, co
 }
 
 // int4: 3 <= M <= 8 from 8.3M weights with 16-bit x (2048 x 4096, M = 4: 9.0 / 7.8; 2048 x 2048: 7.4 /
-// 7.3), 12.5M with F32 x, whose two f16 parts cost twice the conversion (2048 x 4096, M = 4: 9.0 /
+// 7.3), 12M with F32 x, whose two f16 parts cost twice the conversion (2048 x 4096, M = 4: 9.0 /
 // 9.9; 3072 x 4096: 14.8 / 10.2), 16M for rows past 4096 (2048 x 8192, M = 4: 18.1 / 14.5; 1024 x
-// 8192: 10.4 / 14.3).  M > 8 replaces one or two launches more of work that grows with N: BF16 x
-// from 40M (11008 x 4096, M = 12: 24.2 / 20.7; 8192 x 4096: 16.5 / 18.3), 30M past 4096 (4096 x
-// 8192: 17.8 / 16.2); F32 x from 30M (8192 x 4096: 19.5 / 18.4), 16M past 4096 (2048 x 8192: 16.0 /
-// 15.0); F16 x past 4096 only, 16M (2048 x 8192: 16.7 / 14.9; 18944 x 3584: 18.5 / 24.0).
+// 8192: 10.4 / 14.3).  At M <= 4, one pass of the GEMV, it stays the faster one for some rows of 8192 to 17408,
+// where it slows (BF16 x): below 160 tiles from 10240 on (2048 x 14336: 13.9 / 14.9; 2048 x 17152 15.6 / 17.4;
+// x 17408 30.0 / 17.4), from 14336 to 16384 up to three tiles a CU (4608 x 16384: 19.4 / 22.2; 12288 x
+// 15360 32.0 / 29.3), up to 16384 from six on, where a workgroup's tiles take rounds (25600 x 10240: 40.1 / 46.3;
+// 24576 x 10240 35.6 / 34.6).
+// M > 8 replaces one or two launches more of work that grows with N.  F32 x from 30M (8192 x 4096: 19.5 /
+// 18.4), 16M past 4096 (2048 x 8192: 16.0 / 15.0).  BF16 x from 45M (11008 x 4096, M = 12: 24.2 / 20.7; 14336 x
+// 3072, M = 9: 17.8 / 18.9; 8192 x 4096: 16.5 / 18.3); past 4096 30M (4096 x 8192: 17.8 / 16.2), from 18944 on
+// with 192 tiles (3072 x 18944 25.3 / 18.7; 2048 x 18944, G = 256, 19.1 / 20.0).  F16 x past 4096 only, 16M
+// (2048 x 8192: 16.7 / 14.9; 18944 x 3584: 18.5 / 24.0), from 16640 on with 128 tiles (1024 x 18944, G = 256,
+// 17.8 / 19.8), from 22528 on with 192 (2048 x 22528, G = 256, 20.2 / 22.4; 3072 x 28672, 24.5 / 24.1).
 bool skinny_int4_ok(int64_t M, int64_t N, int64_t K, int G, int x_dtype, const void *codes, const void *x) {
   if (M < 3 || M > kSkinnyMaxRows || K <= 0 || K % 128 || K > kSkinnyMaxK || G <= 0 || G % 128 || K % G || N < 1 ||
       (N + 64) * (K / 2) > UINT32_MAX || ((uintptr_t)codes & 15) || ((uintptr_t)x & 15))
     return false;
   const bool lng = K > kSkinnyResMaxK;
-  const int64_t W = N * K, mega = 1000000;
-  if (M <= 8) return W >= (lng ? 16 * mega : x_dtype == F32 ? 12 * mega : 8300000);
-  if (x_dtype == F16) return lng && W >= 16 * mega;
-  return W >= (x_dtype == F32 ? (lng ? 16 : 30) : (lng ? 30 : 40)) * mega;
+  const int64_t W = N * K, mega = 1000000, tiles = cdiv(N, 16);
+  if (M <= 8) {
+    const int64_t cus = device_cus();
+    const bool gemv = M <= 4 && ((K >= 10240 && K < 17408 && tiles < 160) || (K > 14336 && K <= 16384 && tiles <= 3 * cus) ||
+                                 (K > 8192 && K <= 16384 && tiles > 6 * cus));
+    return W >= (lng ? 16 * mega : x_dtype == F32 ? 12 * mega : 8300000) && !gemv;
+  }
+  if (x_dtype == F32) return W >= (lng ? 16 : 30) * mega;
+  if (x_dtype == BF16) return lng ? W >= 30 * mega && (K < 18944 || tiles >= 192) : W >= 45 * mega;
+  return lng && W >= 16 * mega && tiles >= (K < 16640 ? 0 : K < 22528 ? 128 : 192);
 }
 
 size_t skinny_ws_bytes(int64_t M, int64_t K, bool int4) {

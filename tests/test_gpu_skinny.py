@@ -229,6 +229,43 @@ def test_int4(dev, xdt, tol, M, N, K, G):
     assert _err(y, x.double() @ wd.t(), x, wd) <= (tol if M <= 8 else max(tol, 2.0 ** -8 + tol))
 
 
+# Which kernel serves a call shows in its bits: the int8 GEMV gives a row of four the bits it has in a call
+# of two rows, the GEMM a row of nine those it has among seventeen.
+@pytest.mark.parametrize("xdt,M,N,K,G,tiles", [
+    (torch.float32, 4, 2048, 9984, 128, True), (torch.float32, 4, 2048, 10240, 128, False),
+    (torch.float32, 4, 2560, 10240, 128, True), (torch.bfloat16, 4, 2544, 17152, 128, False),
+    (torch.bfloat16, 4, 2048, 17408, 128, True), (torch.float32, 3, 12288, 14464, 128, False),
+    (torch.float32, 3, 12296, 14464, 128, True), (torch.float16, 5, 2048, 14336, 128, True),
+    (torch.bfloat16, 4, 24576, 8320, 128, True), (torch.bfloat16, 4, 24584, 8320, 128, False),
+    (torch.bfloat16, 4, 24584, 8192, 128, True),
+    (torch.bfloat16, 9, 14336, 3072, 128, False), (torch.bfloat16, 16, 11008, 4096, 128, True),
+    (torch.bfloat16, 9, 3056, 18944, 256, False), (torch.bfloat16, 16, 3072, 18944, 256, True),
+    (torch.float16, 9, 1024, 18944, 256, False), (torch.float16, 16, 2048, 18944, 256, True),
+    (torch.float16, 9, 2048, 22528, 256, False), (torch.float16, 16, 3072, 22528, 256, True)])
+def test_int4_takes_the_faster_kernel(dev, xdt, M, N, K, G, tiles):
+    print(f"[case] skinny route int4 x={xdt} M={M} N={N} K={K} G={G}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(K)
+    codes = torch.randint(-2 ** 31, 2 ** 31, (N, K // 8), dtype=torch.int64, device=dev, generator=g).to(torch.int32)
+    s = torch.rand(N, K // G, device=dev, generator=g) * 0.01
+    z = torch.rand(N, K // G, device=dev, generator=g) * 15
+    other = 2 if M <= 8 else 17
+    x = torch.randn(max(M, other), K, device=dev, generator=g).to(xdt)
+    ym, yo = (hipq.int4_matmul(x[:m].contiguous(), codes, s, z, G) for m in (M, other))
+    n = min(M, other)
+    assert torch.equal(ym[:n], yo[:n]) != tiles
+
+
+@pytest.mark.parametrize("dt,N,K,tiles", [(hipq.Q4_K, 24576, 4352, True), (hipq.Q4_K, 24592, 4352, False),
+                                          (hipq.Q5_K, 28656, 4352, False), (hipq.Q5_K, 28672, 4352, True),
+                                          (hipq.Q4_K, 24592, 16640, True), (hipq.Q5_K, 24592, 16640, False)])
+def test_many_long_rows_of_four_take_the_faster_kernel(dev, dt, N, K, tiles):
+    print(f"[case] skinny route dt={hipq.NAMES[dt]} N={N} K={K}", flush=True)
+    w = _big_weight(dt, N, K, dev)
+    x = torch.randn(4, K, device=dev, generator=torch.Generator(device=dev).manual_seed(K))
+    y4, y2 = hipq.matmul_q(x, w, N, K, dt), hipq.matmul_q(x[:2].contiguous(), w, N, K, dt)
+    assert torch.equal(y4[:2], y2) != tiles
+
+
 @pytest.mark.parametrize("dt", [hipq.Q4_K, hipq.Q5_K])
 @pytest.mark.parametrize("M,H,I,gemv", [(3, 2048, 8192, True), (4, 1536, 16384, True), (4, 2048, 16640, False),
                                         (4, 2304, 8192, False), (5, 2048, 8192, False)])

@@ -60,7 +60,8 @@ int workspace(size_t bytes, hipStream_t stream, void **out, const char *call) {
     if (stream && hipStreamIsCapturing(stream, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone)
       return fail(HQ_EUNSUPPORTED, call,
                   "stream is capturing and the library workspace must grow to %zu bytes: pass a workspace", bytes);
-    size_t cap = bytes < (1u << 20) ? (1u << 20) : bytes + bytes / 4;
+    // (The first size serves a captured decode step, weights of any width, after any call on the stream.)
+    size_t cap = bytes < (2u << 20) ? (2u << 20) : bytes + bytes / 4;
     void *p = nullptr;
     if (hipMalloc(&p, cap) != hipSuccess) return fail(HQ_ENOMEM, call, "workspace of %zu bytes", cap);
     if (slot.first) g_ws_retired.push_back({dev, stream, slot.first});

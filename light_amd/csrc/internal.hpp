@@ -107,7 +107,7 @@ bool q4kx_halves_ok(int64_t M, int64_t N, int64_t K, int dt, const void *w, cons
 // The f16 MFMA product for a few rows of x (skinny.hip): Q4_K / Q5_K (w1 != NULL: gated) and
 // int4.  ws: skinny_ws_bytes (rows past 4096 only).
 constexpr int64_t kSkinnyMaxRows = 16;
-// (A row's x record stays below 1 MiB, the library workspace's first size.)
+// (x's records stay below 1 MiB.)
 constexpr int64_t kSkinnyMaxK = 29696;
 bool skinny_ok(int64_t M, int64_t N, int64_t K, int dt, const void *w, const void *x);
 bool skinny_gated_ok(int64_t M, int64_t N, int64_t K, int dt, const void *wg, const void *wu, const void *x);

@@ -1189,9 +1189,14 @@ bool skinny_int4_ok(int64_t M, int64_t N, int64_t K, int G, int x_dtype, const v
   return lng && W >= 16 * mega && tiles >= (K < 16640 ? 0 : K < 22528 ? 128 : 192);
 }
 
+// Two f16 parts of x where the int8 GEMVs keep two levels: rows below 4096 (kX1MinK), and the long
+// rows that gemv_q4kx_kernel's LDS does not take.
+static bool skinny_pair(int64_t K) { return K < 4096 || K > 16384; }
+
 size_t skinny_ws_bytes(int64_t M, int64_t K, bool int4) {
   if (M < 3 || M > kSkinnyMaxRows || K <= kSkinnyResMaxK || K > kSkinnyMaxK) return 0;
-  const int64_t rec = int4 ? 2 * XRec<SkI4, kX16>::BYTES : XRec<SkQk<false>, kX16>::BYTES;
+  const int P = M <= 8 && (int4 || skinny_pair(K)) ? 2 * (int)M : (int)M;  // (int4: as for F32 x)
+  const int64_t rec = int4 ? 2 * XRec<SkI4, kX16>::bytes(P) : XRec<SkQk<false>, kX16>::bytes(P);
   return (size_t)((cdiv(K, 256) * rec + 255) & ~(int64_t)255);
 }
 
@@ -1211,10 +1216,6 @@ static SkinnyArgs skinny_args(const void *x, const void *w, float *out, int64_t 
   a.in_d = act_d_off(M, K);
   return a;
 }
-
-// Two f16 parts of x where the int8 GEMVs keep two levels: rows below 4096 (kX1MinK), and the long
-// rows that gemv_q4kx_kernel's LDS does not take.
-static bool skinny_pair(int64_t K) { return K < 4096 || K > 16384; }
 
 int launch_skinny(const float *x, const void *w0, const void *w1, float *out, int64_t M, int64_t N, int64_t K, int act,
                   int dt, void *ws, hipStream_t s) {

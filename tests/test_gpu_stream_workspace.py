@@ -64,3 +64,33 @@ def test_moe_block_owner_moves_to_next_stream(dev):
         hipq.moe_block_q_check(stream=s)
         assert torch.equal(y, want), rep
         s.destroy()
+
+
+@pytest.mark.parametrize("call", ["gated", "gated_act", "mlp", "matmul"])
+def test_capture_after_a_small_call(dev, call):
+    """A captured call of few rows finds room in the stream's first library workspace, which any small call
+    before the capture has made."""
+    M, N, K = {"gated": (3, 8192, 28672), "gated_act": (3, 14336, 16384), "mlp": (3, 18944, 14336),
+               "matmul": (17, 64, 28672)}[call]
+    print(f"[case] capture after a small call: {call} M={M} N={N} K={K}", flush=True)
+    dt = hipq.Q4_K
+    g = torch.Generator(device=dev).manual_seed(1)
+    w = torch.randint(0, 256, (N * K // 256, 144), dtype=torch.uint8, device=dev, generator=g)
+    w[:, 0:4] = torch.tensor([1e-4, 7e-4], dtype=torch.float16, device=dev).view(torch.uint8)
+    x = torch.randn(M, N if call == "mlp" else K, device=dev, generator=g)
+    run = {"gated": lambda: hipq.matmul_q_gated(x, w, w, N, K, dt), "matmul": lambda: hipq.matmul_q(x, w, N, K, dt),
+           "gated_act": lambda: hipq.matmul_q_act(hipq.matmul_q_gated_act(x, w, w, N, K, dt), w, M, K, N, dt),
+           "mlp": lambda: hipq.mlp_q(x, w, w, w, N, K, dt)}[call]
+    want = run()
+    s, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        hipq.matmul_q(x[:1, :256].contiguous(), w.view(-1)[:144], 1, 256, dt)
+        s.synchronize()
+        with torch.cuda.graph(graph, stream=s):
+            out = run()
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)

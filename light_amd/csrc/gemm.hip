@@ -833,7 +833,7 @@ int gemm_splits(int64_t M, int64_t N, int64_t K) {
 
 size_t gemm_x_bytes(int64_t M, int64_t K) { return ((size_t)M * (size_t)K * 2 + 255) & ~(size_t)255; }
 
-size_t gemm_ws_partial_bytes(int64_t M, int64_t N, int64_t K, bool f32_out);
+size_t gemm_ws_partial_bytes(int64_t M, int64_t N, int64_t K);
 
 // int4 at M <= 64 (gemm_small_int4_kernel): split K until about two workgroups per CU,
 // keeping at least four 128-k stages per split.
@@ -854,7 +854,7 @@ size_t gemm_partial_bytes(int64_t M, int64_t N, int64_t K, bool f32_out) {
     const int s2 = std::max(small_int4_splits(N, K), i4f16_splits(N, K));
     old = std::max(old, (s2 > 1 || !f32_out) ? (size_t)s2 * (size_t)M * (size_t)N * 4 : (size_t)0);
   }
-  return std::max(std::max(old, gemm_ws_partial_bytes(M, N, K, f32_out)), gemm_q4k2_ws_bytes(M, N, K));
+  return std::max(std::max(old, gemm_ws_partial_bytes(M, N, K)), gemm_q4k2_ws_bytes(M, N, K));
 }
 
 static int launch_small_int4(const uint16_t *xb, const uint32_t *codes, const float *sc, const float *zr, void *out,

@@ -24,6 +24,8 @@
 #include "dma.hpp"
 #include "internal.hpp"
 
+#include <type_traits>
+
 namespace hq {
 
 namespace {
@@ -356,8 +358,7 @@ static int ws_splits(int64_t M, int64_t N, int64_t K) {
   return s;
 }
 
-size_t gemm_ws_partial_bytes(int64_t M, int64_t N, int64_t K, bool f32_out) {
-  (void)f32_out;
+size_t gemm_ws_partial_bytes(int64_t M, int64_t N, int64_t K) {
   const int s = ws_splits(M, N, K);
   return s > 1 ? (size_t)s * (size_t)M * (size_t)N * 4 : 0;
 }
@@ -391,7 +392,7 @@ static int launch_ws_t(WsArgs a, int out_dtype, void *out, float *partials, hipS
   a.splits = ws_splits(a.M, a.N, a.K);
   if (a.splits == 1) {
     a.out = out;
-    if constexpr (!WF::DIRECT) {  // (int4: y has x's dtype; the GGUF formats' is F32)
+    if constexpr (std::is_same_v<WF, WsInt4>) {  // (y has x's dtype; the GGUF formats' is F32)
       if (out_dtype == BF16) return launch_ws_o<WF, BM, BF16>(a, s);
       if (out_dtype == F16) return launch_ws_o<WF, BM, F16>(a, s);
     }

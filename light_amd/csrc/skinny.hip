@@ -1118,14 +1118,23 @@ int run_long(SkinnyArgs a, void *ws, hipStream_t s) {
 
 constexpr int64_t kSkinnyResMaxK = 4096;  // longer rows: x prepared in the workspace
 
-template <class F, bool GATED, int XDT, int ODT>
-int run_any(const SkinnyArgs &a, bool pair, void *ws, hipStream_t s) {
-  const bool lng = a.K > kSkinnyResMaxK;
+template <class F, bool GATED, int XM, int XDT, int ODT>
+int run_xm(const SkinnyArgs &a, void *ws, hipStream_t s) {
+  return a.K > kSkinnyResMaxK ? run_long<F, GATED, XM, XDT, ODT>(a, ws, s) : run_resident<F, GATED, XM, XDT, ODT>(a, s);
+}
+
+template <class F, bool GATED, int XDT>
+int run_gguf(const SkinnyArgs &a, bool pair, void *ws, hipStream_t s) {
   if constexpr (XDT >= 0)
-    if (a.M > 8) return lng ? run_long<F, GATED, kX16, XDT, ODT>(a, ws, s) : run_resident<F, GATED, kX16, XDT, ODT>(a, s);
-  constexpr int kPair = XDT == BF16 || XDT == F16 ? kXDup : kXPair;  // (16-bit x needs no second part)
-  if (pair) return lng ? run_long<F, GATED, kPair, XDT, ODT>(a, ws, s) : run_resident<F, GATED, kPair, XDT, ODT>(a, s);
-  return lng ? run_long<F, GATED, kXDup, XDT, ODT>(a, ws, s) : run_resident<F, GATED, kXDup, XDT, ODT>(a, s);
+    if (a.M > 8) return run_xm<F, GATED, kX16, XDT, F32>(a, ws, s);
+  return pair ? run_xm<F, GATED, kXPair, XDT, F32>(a, ws, s) : run_xm<F, GATED, kXDup, XDT, F32>(a, ws, s);
+}
+
+// (16-bit x is exact in one f16 under its unit's scale, down to 2^-24 of the unit's largest element.)
+template <int XDT>
+int run_int4(const SkinnyArgs &a, void *ws, hipStream_t s) {
+  if (a.M > 8) return run_xm<SkI4, false, kX16, XDT, XDT>(a, ws, s);
+  return run_xm<SkI4, false, XDT == F32 ? kXPair : kXDup, XDT, XDT>(a, ws, s);
 }
 
 }  // namespace
@@ -1225,8 +1234,8 @@ int launch_skinny(const float *x, const void *w0, const void *w1, float *out, in
   a.xdt = F32;
   const bool pair = skinny_pair(K);
   if (dt == Q5_K)
-    return w1 ? run_any<SkQk<true>, true, F32, F32>(a, pair, ws, s) : run_any<SkQk<true>, false, F32, F32>(a, pair, ws, s);
-  return w1 ? run_any<SkQk<false>, true, F32, F32>(a, pair, ws, s) : run_any<SkQk<false>, false, F32, F32>(a, pair, ws, s);
+    return w1 ? run_gguf<SkQk<true>, true, F32>(a, pair, ws, s) : run_gguf<SkQk<true>, false, F32>(a, pair, ws, s);
+  return w1 ? run_gguf<SkQk<false>, true, F32>(a, pair, ws, s) : run_gguf<SkQk<false>, false, F32>(a, pair, ws, s);
 }
 
 int launch_skinny_act(const void *x, const void *w, float *out, int64_t M, int64_t N, int64_t K, int dt, void *ws,
@@ -1234,7 +1243,7 @@ int launch_skinny_act(const void *x, const void *w, float *out, int64_t M, int64
   SkinnyArgs a = skinny_args(x, w, out, M, N, K, dt);
   a.xdt = kXAct;
   const bool pair = skinny_pair(K);
-  return dt == Q5_K ? run_any<SkQk<true>, false, kXAct, F32>(a, pair, ws, s) : run_any<SkQk<false>, false, kXAct, F32>(a, pair, ws, s);
+  return dt == Q5_K ? run_gguf<SkQk<true>, false, kXAct>(a, pair, ws, s) : run_gguf<SkQk<false>, false, kXAct>(a, pair, ws, s);
 }
 
 // ---- 17 <= M <= 64, Q4_K / Q5_K (skinny_mid_kernel) ----
@@ -1321,10 +1330,10 @@ int launch_skinny_int4(const void *x, int x_dtype, const uint32_t *codes, const 
   a.tiles = (int)cdiv(N, 16);
   a.row_bytes = (uint32_t)(K / 2);
   a.last = (uint32_t)(N * a.row_bytes - 16);
-  switch (x_dtype) {  // (BF16 and F16 x are exact in one f16 under the unit's scale)
-    case F32: return run_any<SkI4, false, F32, F32>(a, true, ws, s);
-    case BF16: return run_any<SkI4, false, BF16, BF16>(a, false, ws, s);
-    case F16: return run_any<SkI4, false, F16, F16>(a, false, ws, s);
+  switch (x_dtype) {
+    case F32: return run_int4<F32>(a, ws, s);
+    case BF16: return run_int4<BF16>(a, ws, s);
+    case F16: return run_int4<F16>(a, ws, s);
     default: return fail(HQ_EUNSUPPORTED, "int4_matmul", "x dtype %d", x_dtype);
   }
 }

@@ -255,3 +255,24 @@ def test_prefill_weights_are_s_times_q_minus_z(dev, xdt, M, N, K):
     y = hipq.int4_matmul(x, _t(codes, dev).view(torch.int32), _t(s, dev), _t(z, dev), 64)
     want = -x[:, torch.from_numpy(c).to(dev)].float() * _t(s[n, c // 64], dev).to(torch.bfloat16).float()
     assert torch.equal(y, want.to(TDT[xdt]))
+
+
+@pytest.mark.parametrize("xdt", [hipq.F32, hipq.BF16, hipq.F16])
+@pytest.mark.parametrize("M,N,K,G", [(65, 257, 960, 64), (129, 131, 448, 64), (128, 33001, 512, 128), (300, 8321, 1024, 256),
+                                     (1000, 5001, 2048, 128)])
+def test_prefill_tiles_store_every_dtype(dev, xdt, M, N, K, G):
+    """One K part (K < 1024, or tiles enough to fill the chip): the tiles store y in x's dtype themselves.
+    x (F32, F16) and w are each rounded once to bf16 (2^-8), y once to its dtype; the f32 sums add K 2^-24."""
+    print(f"[case] int4 one part M={M} N={N} K={K} G={G} x={hipq.NAMES[xdt]}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(N)
+    codes = torch.randint(-2 ** 31, 2 ** 31, (N, K // 8), dtype=torch.int64, device=dev, generator=g).to(torch.int32)
+    s = torch.rand(N, K // G, device=dev, generator=g) * 0.02 + 1e-3
+    z = torch.rand(N, K // G, device=dev, generator=g) * 15
+    x = torch.randn(M, K, device=dev, generator=g).to(TDT[xdt])
+    y = hipq.int4_matmul(x, codes, s, z, G)
+    wd = hipq.int4_dequant(codes, s, z, G).double()
+    want = x.double() @ wd.t()
+    operands = (2.0 ** -8 if xdt == hipq.BF16 else 2.0 ** -7) + K * 2.0 ** -24
+    bound = operands * (x.double().abs() @ wd.abs().t()) + ULP[xdt] * want.abs()
+    assert ((y.double() - want).abs() <= bound * 1.02).all()  # (1.02: the roundings' products)
+    assert torch.equal(y, hipq.int4_matmul(x, codes, s, z, G)), "not deterministic"

@@ -111,8 +111,9 @@ size_t hq_matmul_q_ws_bytes(int64_t M, int64_t N, int64_t K, int w_dtype);
  * w_dtype: one of the six GGUF formats Light fuses: HQ_Q4_0, HQ_Q5_0, HQ_Q8_0, HQ_Q4_K,
  * HQ_Q5_K or HQ_Q6_K, or HQ_Q6_K_R (a Q6_K weight after hq_repack_q6k).  K must be a
  * multiple of the block size.
- *  - 3 <= M <= 64, Q4_K / Q5_K (from about 10M weights at M <= 8): f16 MFMA on exact integer weights,
- *    x as one or two f16 parts under a power-of-two scale per row and 256 elements.
+ *  - 3 <= M <= 64, Q4_K / Q5_K, K <= 29696 (at M <= 8 from 10M weights, and past K = 4096 from 1536 columns
+ *    and, at M <= 4, where the tiles fill the chip): f16 MFMA on exact integer weights, x as one or two f16
+ *    parts under a power-of-two scale per row and 256 elements.
  *  - Other M <= 8, Q4_K / Q5_K / Q6_K_R: the persistent int8-dot GEMV, x quantized to q8_1 inside its
  *    workgroups (K > 8192: into ws first).
  *  - M <= 8, Q8_0 / Q4_0 / Q5_0 / Q6_K: the LDS-staged int8-dot GEMV (x quantized in its
@@ -167,11 +168,12 @@ int hq_matmul_q_gated(const float *x, const void *wg, const void *wu, float *out
 /* Gated projection that emits prepared activations for the next matmul:
  *   act_out (hq_act_bytes(M, N) bytes) = quantize_act(act(x @ dequant(wg)^T) * (x @ dequant(wu)^T)),
  * the same values hq_quantize_act would write for the F32 gated output.  N % 32 == 0.
- * For Q4_K / Q5_K with M <= 2 (and small weights to M <= 8) this is one kernel: the gated GEMV
- * quantizes each completed 32-row chunk of its output in the epilogue (the first launch of
- * hq_mlp_q).  Other cases run hq_matmul_q_gated into ws, then the quantizer.  Feed act_out to hq_matmul_q_act (the
- * down projection).  Light: models/llama.go:1306-1328 (gate, up, SiLU * up before
- * DownProj); no counterpart op in Light. */
+ * For Q4_K / Q5_K whose projections take the gated int8 GEMV (M <= 2; M <= 4 but for 10M weights and more of
+ * 2048 < K <= 4096; M <= 8 with fewer than 10M weights, past K = 4096 with fewer than 1536 rows too, or past
+ * K = 29696) and N % 256 == 0 this is one kernel: that GEMV quantizes each completed 32-row chunk of its output
+ * in the epilogue (the first launch of hq_mlp_q).  Other cases run hq_matmul_q_gated into ws, then the quantizer.
+ * Feed act_out to hq_matmul_q_act (the down projection).  Light: models/llama.go:1306-1328 (gate, up, SiLU * up
+ * before DownProj); no counterpart op in Light. */
 size_t hq_matmul_q_gated_act_ws_bytes(int64_t M, int64_t N, int64_t K, int w_dtype);
 int hq_matmul_q_gated_act(const float *x, const void *wg, const void *wu, void *act_out, int64_t M, int64_t N,
                           int64_t K, int w_dtype, int act, void *ws, size_t ws_bytes, hq_stream_t stream);
@@ -179,11 +181,11 @@ int hq_matmul_q_gated_act(const float *x, const void *wg, const void *wu, void *
 /* The gated MLP block of a decoder layer:
  *   out (M, H) F32 = (act(x @ dequant(wg)^T) * (x @ dequant(wu)^T)) @ dequant(wd)^T
  * with x (M, H) F32, wg and wu (I, H), wd (H, I), all of w_dtype; act as above.
- * For Q4_K / Q5_K with M <= 8 whose gate/up takes the int8 GEMV (M <= 2, small weights, other rows at
- * M <= 4 than 2048 < H <= 4096) that GEMV writes h already quantized for the next matmul into ws, as
- * hq_matmul_q_gated_act does, and the down projection runs on it: hq_matmul_q_act, bit for bit, or at
- * M >= 3 past I = 4096 its f16 MFMA form.  Other cases run hq_matmul_q_gated into ws and then hq_matmul_q,
- * bit for bit.
+ * For Q4_K / Q5_K with M <= 8 whose gate/up takes the int8 GEMV (as above) that GEMV writes h already
+ * quantized for the next matmul into ws, as hq_matmul_q_gated_act does, and the down projection runs on
+ * it: hq_matmul_q_act, bit for bit, or at M >= 3 past I = 4096 its f16 MFMA form.  Other cases run
+ * hq_matmul_q_gated into ws and then hq_matmul_q, bit for bit (M > 8, both on the bf16 GEMM: h goes straight
+ * to the bf16 that the down projection would round it to).
  * Light: models/llama.go:1306-1333 (GatedLinear or MatMulQ/SiLU/Mul, then DownProj).
  * No counterpart op in Light. */
 size_t hq_mlp_q_ws_bytes(int64_t M, int64_t H, int64_t I, int w_dtype);
@@ -192,7 +194,8 @@ int hq_mlp_q(const float *x, const void *wg, const void *wu, const void *wd, flo
 
 /* Prepared activations: hq_matmul_q = hq_quantize_act + hq_matmul_q_act (bit for bit
  * for Q8_0 / Q6_K; the Q4_K GEMV quantizes x inside its own workgroups with
- * reciprocal-based scales, so there the two agree to the activation rounding).
+ * reciprocal-based scales, and past two rows hq_matmul_q can take the f16 MFMA form, so
+ * there the two agree to the activation rounding).
  * A caller that multiplies one activation by several weights (the SwiGLU gate
  * and up projections, models/llama.go:1306-1328) quantizes once and reuses it.
  * No counterpart in Light.  The act buffer (hq_act_bytes(M, K) bytes, 16-byte
@@ -259,8 +262,9 @@ size_t hq_int4_matmul_ws_bytes(int64_t M, int64_t N, int64_t K, int G, int x_dty
  * quant/int4.go:11-34): codes U32 (N, K/8), nibble j of word c = W[n, 8c+j];
  * scales / zeros F32 (N, K/G); W = s * (code - z).  x_dtype F32, BF16 or F16;
  * y has x's dtype (F16 is an extension: Light takes F32 or BF16, ops/int4.go:70-72).
- * K % 32 == 0 and G % 32 == 0.  3 <= M <= 16, G % 128 == 0 and large weights: f16 MFMA on the exact
- * codes, F32 x as two f16 parts (16-bit x is exact in one).  Other M <= 8 (or G % 64 != 0): x is quantized to q8_1
+ * K % 32 == 0 and G % 32 == 0.  3 <= M <= 16, G % 128 == 0, K <= 29696 and large weights: f16 MFMA on the
+ * exact codes, F32 x as two f16 parts (one above M = 8; 16-bit x is exact in one, down to 2^-24 of the largest
+ * of its 128 elements).  Other M <= 8 (or G % 64 != 0): x is quantized to q8_1
  * into ws and the int8-dot GEMV runs (K <= 65536; rows past 32768 with 256 % G == 0 as two
  * K halves whose F32 partials are summed in ws); otherwise -- and for longer rows at
  * any M when G % 64 == 0 -- the MFMA GEMMs run (F16 x at 8 < M <= 64 as given, else

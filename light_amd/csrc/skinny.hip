@@ -6,21 +6,22 @@
 // a speculative step, where each weight is used M times.
 //
 // The int8-dot GEMV pays its dot products, scale arithmetic and a re-read of the weights (four
-// rows of x per pass) once per row: at M = 6 it is VALU-bound (gate/up 14336 x 4096, Q4_K:
-// 60.8 us for 66 MB, down 4096 x 14336 30.4 us; here 20.5 and 13.3 us, plus 4.8 us for the long
-// rows' x).  A wave multiplies a tile of 16 weight rows by up to 16 rows of x with
-// v_mfma_f32_16x16x32_f16, so the weight bytes are unpacked once whatever M is.  What bounds it
-// now: the unpacking (about nine VALU instructions per eight weights and lane, 18 of the 23 us
-// remain without it), and for the long rows the records of x, which every CU reads from L2
-// (13.3 us, 9.4 us without them).
+// rows of x per pass) once per row.  A wave here multiplies a tile of 16 weight rows by up to 16 rows of
+// x with v_mfma_f32_16x16x32_f16, so the weight bytes are unpacked once whatever M is.  Q4_K, M = 6,
+// layers replayed from a graph, that GEMV / this: gate/up 14336 x 4096 46.9 / 21.2 us (66 MB), down
+// 4096 x 14336 33.1 / 16.8 (33 MB, the launch for the long rows' x among them).
+// What bounds it now, by counters of these calls.  Gate/up: VALU issues on 60 % of a SIMD's cycles (3.4
+// instructions per weight and lane; the unpacking's nine per eight weights are a third of them), MFMA
+// is busy on a tenth, LDS bank conflicts fill a quarter of a CU's.  Down: VALU 37 %, MFMA 7 %; seven of
+// ten requests to L2 are not for weights but for the records of x, which every CU reads, and waves wait.
 //  * B holds exact integers in f16: sc * q (6-bit scale times quant, at most 63 * 31) for the K
 //    formats, q for int4.  A nibble pair becomes (1024 + q) by one v_and_or_b32, and one packed
 //    FMA by (sc, -1024 sc) leaves sc * q without rounding (high nibbles in place: 1024 + 16 q
 //    with sc / 16).  d, dmin, s and z stay f32 and are applied to the f32 sums of a unit.
 //  * A holds x as f16 under a power-of-two scale per row and unit (256 elements; int4 128), so
-//    no x overflows or loses its small elements.  XM = kXPair (M <= 8) splits x into two f16
-//    (rows 0-7 the high parts, rows 8-15 the remainders): 22 bits, for the calls whose int8
-//    form keeps two levels.  XM = kXDup (M <= 8): rows 8-15 repeat rows 0-7, one f16 level
+//    no x overflows and no element down to 2^-24 of its unit's largest is lost.  XM = kXPair (M <= 8)
+//    splits x into two f16 (rows 0-7 the high parts, rows 8-15 the remainders): 22 bits, for the calls
+//    whose int8 form keeps two levels.  XM = kXDup (M <= 8): rows 8-15 repeat rows 0-7, one f16 level
 //    (2^-12, against 2^-8 of q8_1's single level).  XM = kX16: sixteen rows, one level.
 //  * The lane group g = lane / 16 of a fragment holds the unit's g-th quarter (Q4_K: pair g),
 //    so a lane unpacks only its own quarter's scales.  The minimum term is one more MFMA per
@@ -896,8 +897,9 @@ __global__ __launch_bounds__(256) void skinny_x_kernel(SkinnyArgs a, uint8_t *xf
 // added by splitk_reduce_kernel).  All waves multiply the same unit, so x's record (up to 64 rows,
 // 34 KB) is staged in LDS once per workgroup, and each unpacked weight fragment meets MT of its
 // row tiles.  Per unit: wait for this wave's direct loads, one barrier, request the next unit, work.
-// Against the bf16 GEMM of 64-row tiles, whose f32 dequantization (3.5 VALU instructions per
-// weight against 1.4 here) bounds it.
+// What bounds it, by counters of 14336 x 4096 at M = 40: no unit alone -- VALU issues on 40 % of a SIMD's
+// cycles, MFMA is busy on 19 %, LDS on a third of a CU's with its bank conflicts -- but the chain through
+// them with two waves a SIMD.
 template <class F>
 struct SkinnyMidLds {
   static constexpr int WST = (16 * F::BB + 1023) / 1024 * 1024;  // a wave's weights of one unit
@@ -1140,19 +1142,22 @@ int run_int4(const SkinnyArgs &a, void *ws, hipStream_t s) {
 }  // namespace
 
 // Where this file's kernels are the faster ones (us per call, the int8 GEMV or the GEMMs against
-// them; layers replayed from a graph, Q4_K unless named):
-//  * M = 2: the GEMV reads the weights once for both rows (14336 x 4096: 11.3 / 13.2).
-//  * 3 <= M <= 8: from 10M weights (2560 x 4096, M = 3: 10.6 / 7.6; M = 8: 14.5 / 9.3; 2048 x 4096,
-//    M = 3: 7.2 / 7.5).  Below, the GEMV's one pass of two row groups per CU beats the conversion
-//    of x (2048 x 2048, M = 3: 6.9 / 9.2).  Rows past 4096 prepare x in a launch of its own and
-//    need 96 tiles (1536 x 14336, M = 3: 15.2 / 14.4; 1024 x 16384: 11.4 / 16.2).
-//  * Gated at M <= 4: rows of (2048, 4096] only (the MLP of 2048 x 8192 at M = 3: 21.9 / 25.1 with
-//    both halves here; 4096 x 14336: 51.8 / 38.1).
+// them; layers of more than 600 MB replayed from a graph, a path that the rule does not take and shapes of
+// more than 100M weights: of fewer layers; Q4_K unless named):
+//  * M = 2: the GEMV reads the weights once for both rows (14336 x 4096: 10.2 / 13.2).
+//  * 3 <= M <= 8: from 10M weights (2560 x 4096, M = 3: 9.6 / 6.6; M = 8: 13.3 / 8.3; 2048 x 4096,
+//    M = 3: 6.2 / 7.5).  Below, the GEMV's one pass of two row groups per CU beats the conversion
+//    of x (2048 x 2048, M = 3: 6.1 / 9.2).  Rows past 4096 prepare x in a launch of its own and
+//    need 96 tiles (1536 x 14336, M = 3: 14.9 / 14.3; 1024 x 16384: 10.1 / 16.2).
+//  * Gated at M <= 4: rows of (2048, 4096] only (the MLP of 2048 x 8192 at M = 3: 21.0 / 25.1 with
+//    both halves here; 4096 x 14336: 52.0 / 37.1).
 //    At M <= 4, one pass of the GEMV, past six tiles a CU only where the rounds of workgroups are nearly full
 //    (28672 x 8192 39.6 / 36.7; 25600 x 16384 54.0 / 58.1; 50426 x 4864 42.7 / 50.4), or Q4_K past 16384,
 //    where its GEMV slows (24576 x 18944: 146.5 / 70.2).
 //  * M > 8: always, against the GEMM's conversion, product and split-K launches (14336 x 4096,
-//    M = 12: 30.6 / 20.1; 1024 x 4096: 16.1 / 13.8).
+//    M = 12: 29.3 / 19.4; 1024 x 4096, M = 9: 14.9 / 12.7), few columns of long rows too, where this does
+//    not split K and the GEMM does: 32 to 1536 rows of 2048 to 28672, Q4_K and Q5_K, M = 9 and 16, all
+//    faster but Q5_K, 32 x 28672 at M = 16 (20.1 / 21.4; 128 x 28672 28.7 / 22.1).
 bool skinny_ok(int64_t M, int64_t N, int64_t K, int dt, const void *w, const void *x) {
   if ((dt != Q4_K && dt != Q5_K) || M < 3 || M > kSkinnyMaxRows || K <= 0 || K % 256 || K > kSkinnyMaxK || N < 1 ||
       (N + 64) * (K / 256) * block_info(dt).bytes > UINT32_MAX || ((uintptr_t)w & 15) || ((uintptr_t)x & 15))
@@ -1259,10 +1264,11 @@ static int mid_splits(int64_t N, int64_t K) {
   return (int)s;
 }
 
-// Every such call (us, the bf16 GEMM with its conversion and reduce / this; Q4_K): 14336 x 4096 M = 24 28.2 /
-// 17.4, M = 40 28.7 / 22.9, M = 64 30.0 / 27.1; 4096 x 14336 M = 64 36.4 / 26.5; 512 x 1024 M = 20 13.7 / 8.9;
-// 28672 x 8192 M = 40 94.7 / 63.7.  Q5_K, which the GEMM first expands to bf16 in memory: 14336 x 4096 M = 40
-// 94.1 / 23.4.
+// Every such call (us, the bf16 GEMM with its conversion and reduce / this; layers of more than 600 MB
+// replayed from a graph, Q4_K): 14336 x 4096 M = 17 29.6 / 18.9, M = 24 30.0 / 19.5, M = 40 31.1 / 22.1, M = 64
+// 32.6 / 26.0; 4096 x 14336 M = 64 39.8 / 26.5; 512 x 1024 M = 20 13.5 / 8.6; 28672 x 8192 M = 40 96.5 / 62.4.
+// Q5_K, which the GEMM first expands to bf16 in memory: 14336 x 4096 M = 40 78.9 / 24.1.  32 to 1536 rows of
+// 2048 to 28672 at M = 17, 33 and 64: all faster but Q5_K, 32 x 28672 at M = 64 (23.0 / 23.3).
 bool skinny_mid_ok(int64_t M, int64_t N, int64_t K, int dt, const void *w, const void *x) {
   return (dt == Q4_K || dt == Q5_K) && M > kSkinnyMaxRows && M <= 64 && K > 0 && K % 256 == 0 && K <= kSkinnyMaxK && N >= 1 &&
          N * (K / 256) * block_info(dt).bytes <= UINT32_MAX && ((uintptr_t)w & 15) == 0 && ((uintptr_t)x & 15) == 0;

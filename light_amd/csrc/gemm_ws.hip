@@ -142,10 +142,11 @@ struct WsInt4 {
     const float s = reinterpret_cast<const float *>(raw + 1024)[r];
     const float z = reinterpret_cast<const float *>(raw + 1024)[32 + r];
     // The exact weight s (q - z), rounded once to f32 and once to bf16; the quants as bytes (one mask
-    // per four, v_cvt_f32_ubyteN).
+    // per four, v_cvt_f32_ubyteN; the empty asm keeps the compiler from a bit-field extract each).
 #pragma unroll
     for (int k = 0; k < 4; k++) {
-      const uint32_t ev = q[k] & 0x0F0F0F0Fu, od = (q[k] >> 4) & 0x0F0F0F0Fu;
+      uint32_t ev = q[k] & 0x0F0F0F0Fu, od = (q[k] >> 4) & 0x0F0F0F0Fu;
+      asm("" : "+v"(ev), "+v"(od));
 #pragma unroll
       for (int j = 0; j < 8; j++) {
         const float v = s * ((float)((((j & 1) ? od : ev) >> (8 * (j >> 1))) & 0xffu) - z);
